@@ -735,8 +735,13 @@ void Engine::pack() {
     check_hip(hipMemset(d_.scan_total, 0, 2 * sizeof(int)), "memset");
     d_.types_f = dalloc<float>(types_f.size()); upload(d_.types_f, types_f);
     d_.types_d = dalloc<double>(types_d.size()); upload(d_.types_d, types_d);
-    d_.energy = dalloc<long long>(static_cast<size_t>(nsys) * 32);
-    d_.ke = dalloc<long long>(nsys);
+    // copies of the energy words spread the atomics: one per 256 member rows
+    // of a system, up to 64 (many systems spread over words of their own, and
+    // a small system's few atomics cost less than the launch that sums copies)
+    d_.ecopies = 1;
+    while (d_.ecopies < 64 && d_.ecopies * 2 * 256 <= d_.nm / nsys) d_.ecopies *= 2;
+    d_.estride = (nsys * 33 + 31) & ~31;
+    d_.energy = dalloc<long long>(static_cast<size_t>(d_.ecopies) * d_.estride);
     d_.dump_count = dalloc<int>(1);
     int team = opt_.team_size;
     if (team != 4 && team != 8 && team != 16 && team != 32 && team != 64) team = 16;
@@ -1474,6 +1479,7 @@ std::vector<double> Engine::potentials() {
     launch_zero_energy(d_, stream_);
     launch_bonded(d_, stream_, true, d_.f2, 0xFFFFFFFFu);
     launch_pair(d_, stream_, true, d_.f2, 0xFFFFFFFFu);
+    launch_energy_reduce(d_, stream_);
     sync();
     check_hip(hipMemsetAsync(d_.err, 0, sizeof(int) * d_.nsys, stream_), "memset");
     std::vector<long long> e(static_cast<size_t>(d_.nsys) * 32);
@@ -1711,6 +1717,7 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
         launch_bonded(d_, stream_, true, d_.f2, groups);
         launch_pair(d_, stream_, true, d_.f2, groups);
         launch_kinetic(d_, stream_);
+        launch_energy_reduce(d_, stream_);
         sync();
         check_hip(hipMemsetAsync(d_.err, 0, sizeof(int) * d_.nsys, stream_), "memset");   // energies raise no step error
         int flags = 0;
@@ -1724,7 +1731,7 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
         std::vector<long long> e(32);
         long long ke = 0;
         check_hip(hipMemcpy(e.data(), d_.energy + static_cast<size_t>(s) * 32, 32 * sizeof(long long), hipMemcpyDeviceToHost), "energy");
-        check_hip(hipMemcpy(&ke, d_.ke + s, sizeof(long long), hipMemcpyDeviceToHost), "ke");
+        check_hip(hipMemcpy(&ke, d_.energy + static_cast<size_t>(d_.nsys) * 32 + s, sizeof(long long), hipMemcpyDeviceToHost), "ke");
         out->potential_energy = 0;
         for (int g = 0; g < 32; ++g) {
             out->energy_by_group[g] = e[g] * kFixInv;

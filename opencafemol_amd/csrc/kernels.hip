@@ -15,7 +15,7 @@
 //   k_snapshot / k_status_out   chunk start snapshot and end-of-chunk flags
 // Forces are computed in FP32 from FP64 displacements and accumulated as
 // 64-bit fixed point (2^-32 kJ/mol/nm); positions/velocities are FP64.
-// The energy pass (k_pair / k_bonded with ENERGY=true) evaluates terms in FP64.
+// The energy pass (k_pair_energy, k_bonded<true>, k_kinetic) evaluates terms in FP64.
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -1193,9 +1193,10 @@ __global__ void k_bonded(int nt, const BTerm* __restrict__ terms, const DevSys* 
                          const int* __restrict__ sys_of, const double* __restrict__ px,
                          const double* __restrict__ py, const double* __restrict__ pz,
                          const FlaTable* __restrict__ fla, const FldTable* __restrict__ fld,
-                         ForceOut out, long long* __restrict__ energy, uint32_t groups,
+                         ForceOut out, long long* __restrict__ energy, int ecopies, int estride, uint32_t groups,
                          int* __restrict__ err) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (ENERGY) energy += static_cast<size_t>(blockIdx.x & (ecopies - 1)) * estride;
     long long ef = 0;
     int key = -1;   // energy word of this term (ENERGY)
     if (t < nt) {
@@ -1670,6 +1671,15 @@ __device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const 
     return static_cast<double>(gg * 4294967296.0f);
 }
 
+// The kinds of a group whose energy group is in the mask.
+__device__ __forceinline__ int group_kinds(const DevPairGroup& G, uint32_t gmask) {
+    int kinds = 0;
+#pragma unroll
+    for (int k = 0; k < kPairKinds; ++k)
+        if (((G.kinds >> k) & 1) && ((gmask >> G.egroup[k]) & 1u)) kinds |= 1 << k;
+    return kinds;
+}
+
 // The pair kernel's spec (specialized row loop) of a group with these kinds.
 __device__ __forceinline__ int pair_spec(int kinds, bool periodic, const PairK<float>& Kf) {
     if (kinds == kExv) return periodic ? kSpecExvPeriodic : kSpecExvOpen;
@@ -1888,13 +1898,13 @@ __global__ __launch_bounds__(kPairBlock) void k_prune(int nm, const DevPairGroup
 
 // At least 5 waves per SIMD (<= 96 VGPRs): the record gathers need the latency hiding.
 // SLICED: walk the table in XCD slices (xcd_walk); otherwise a plain stride.
-template <bool ENERGY, int TEAM, bool SLICED, int U>
+template <int TEAM, bool SLICED, int U>
 __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_pair(
     const DevPairGroup* __restrict__ groups, const int2* __restrict__ blocks,
     const PairRec* __restrict__ rec, const int* __restrict__ row_start,
     const int* __restrict__ row_count, const int* __restrict__ col,
-    const float* __restrict__ types_f, const double* __restrict__ types_d, ForceBuf out,
-    long long* __restrict__ energy, uint32_t gmask, int* __restrict__ err, int nblocks, int nrec,
+    const float* __restrict__ types_f, ForceBuf out,
+    uint32_t gmask, int* __restrict__ err, int nblocks, int nrec,
     unsigned long long* __restrict__ stamp, BondedArgs bd) {
     extern __shared__ __attribute__((aligned(16))) float lds_types[];
     int loaded = -1;
@@ -1908,19 +1918,17 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
     for (int bi = walk.first; bi < walk.end; bi += walk.stride) {
     const int2 bt = blocks[bi];
     if (bt.x < 0) {
-        // a chunk of bonded terms, one per thread (force pass only): their
-        // gathers and atomics overlap the pair rows of the other workgroups
-        if (!ENERGY) {
-            const int t = bt.y + static_cast<int>(threadIdx.x);
-            if (t < bd.nt) {
-                const BTerm T = bd.terms[t];
-                if ((gmask >> (T.meta & 31)) & 1u) {
-                    const int s = bd.sys_of[T.idx[0]];
-                    int bad = 0;
-                    bonded_term<false, float>(T, bd.sys[s], bd.px, bd.py, bd.pz, bd.fla, bd.fld,
-                                              ForceOut{out.fx, out.fy, out.fz}, nullptr, s, bad);
-                    if (bad) atomicOr(&err[s], kErrNumeric);
-                }
+        // a chunk of bonded terms, one per thread: their gathers and atomics
+        // overlap the pair rows of the other workgroups
+        const int t = bt.y + static_cast<int>(threadIdx.x);
+        if (t < bd.nt) {
+            const BTerm T = bd.terms[t];
+            if ((gmask >> (T.meta & 31)) & 1u) {
+                const int s = bd.sys_of[T.idx[0]];
+                int bad = 0;
+                bonded_term<false, float>(T, bd.sys[s], bd.px, bd.py, bd.pz, bd.fla, bd.fld,
+                                          ForceOut{out.fx, out.fy, out.fz}, nullptr, s, bad);
+                if (bad) atomicOr(&err[s], kErrNumeric);
             }
         }
         continue;
@@ -1929,119 +1937,64 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
     const RowGeom geo{G.box[0], G.box[1], G.box[2], G.inv_box[0], G.inv_box[1], G.inv_box[2], G.rc2, G.rin2,
                       G.periodic != 0};
     const PairK<float> Kf = pair_constants<float>(G);
-    const PairK<double> Kd = pair_constants<double>(G);
-    if (!ENERGY && bt.x != loaded) {  // bt.x is uniform over the workgroup
+    if (bt.x != loaded) {  // bt.x is uniform over the workgroup
         __syncthreads();
         const float* src = types_f + static_cast<size_t>(G.type_begin) * kTypeStride;
         for (int k = threadIdx.x; k < G.n_types * kTypeStride; k += blockDim.x) lds_types[k] = src[k];
         __syncthreads();
         loaded = bt.x;
     }
-    int kinds = 0;
-#pragma unroll
-    for (int k = 0; k < kPairKinds; ++k)
-        if (((G.kinds >> k) & 1) && ((gmask >> G.egroup[k]) & 1u)) kinds |= 1 << k;
+    const int kinds = group_kinds(G, gmask);
     const int lane = threadIdx.x % TEAM;
     const int row = bt.y + threadIdx.x / TEAM;
     const int row_end = G.member_begin + G.member_count;
     RowAcc acc;
-    long long ae0 = 0, ae1 = 0, ae2 = 0, ae3 = 0;
     int bead_i = -1;
     if (row < row_end && kinds) {
         const PairRec ri = rec[row];
         bead_i = ri.bead;
         const int beg = row_start[row], cnt = row_count[row];
         const int ti = ri.type & 0xFFFF;
-        if (!ENERGY) {
-            const RowType rt = row_type(lds_types + ti * kTypeStride);
-            // the group's kind selects the loop (uniform over the workgroup)
-            switch (pair_spec(kinds, geo.periodic, Kf)) {
-            case kSpecExvPeriodic:
-                force_row<TEAM, kSpecExvPeriodic, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                         lds_types, acc);
-                break;
-            case kSpecExvOpen:
-                force_row<TEAM, kSpecExvOpen, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                     lds_types, acc);
-                break;
-            case kSpecDh:
-                force_row<TEAM, kSpecDh, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                lds_types, acc);
-                break;
-            case kSpecLjShared:
-                force_row<TEAM, kSpecLjShared, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                      lds_types, acc);
-                break;
-            case kSpecSolo:
-                force_row<TEAM, kSpecSolo, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                  lds_types, acc);
-                break;
-            default:
-                force_row<TEAM, kSpecGeneric, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                     lds_types, acc);
-                break;
-            }
-        } else {
-            // energy pass: FP64 terms of each pair once (row < column)
-            const double* tdi = types_d + static_cast<size_t>(G.type_begin + ti) * kTypeStride;
-            const int4* col4 = reinterpret_cast<const int4*>(col + beg);
-            for (int k = lane; 4 * k < cnt; k += TEAM) {
-                const int4 c4 = col4[k];
-                const int cs[4] = {c4.x, c4.y, c4.z, c4.w};
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const int s = cs[u];
-                    if (s < 0 || row >= s) continue;
-                    const PairRec rj = rec[s];
-                    double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
-                    if (geo.periodic) {
-                        dx = min_image(dx, geo.bx, geo.ibx);
-                        dy = min_image(dy, geo.by, geo.iby);
-                        dz = min_image(dz, geo.bz, geo.ibz);
-                    }
-                    const double r2 = dist2(dx, dy, dz);
-                    if (!(r2 < geo.rc2)) continue;
-                    double f;
-                    double e[4] = {0, 0, 0, 0};
-                    const double* tdj = types_d + static_cast<size_t>(G.type_begin + (rj.type & 0xFFFF)) * kTypeStride;
-                    pair_eval<double>(kinds, Kd, nullptr, nullptr, tdi, tdj, r2, &f, e);
-                    ae0 += to_fix_d(e[0], acc.bad);
-                    ae1 += to_fix_d(e[1], acc.bad);
-                    ae2 += to_fix_d(e[2], acc.bad);
-                    ae3 += to_fix_d(e[3], acc.bad);
-                }
-            }
+        const RowType rt = row_type(lds_types + ti * kTypeStride);
+        // the group's kind selects the loop (uniform over the workgroup)
+        switch (pair_spec(kinds, geo.periodic, Kf)) {
+        case kSpecExvPeriodic:
+            force_row<TEAM, kSpecExvPeriodic, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
+                                                 lds_types, acc);
+            break;
+        case kSpecExvOpen:
+            force_row<TEAM, kSpecExvOpen, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
+                                             lds_types, acc);
+            break;
+        case kSpecDh:
+            force_row<TEAM, kSpecDh, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
+                                        lds_types, acc);
+            break;
+        case kSpecLjShared:
+            force_row<TEAM, kSpecLjShared, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
+                                              lds_types, acc);
+            break;
+        case kSpecSolo:
+            force_row<TEAM, kSpecSolo, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
+                                          lds_types, acc);
+            break;
+        default:
+            force_row<TEAM, kSpecGeneric, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
+                                             lds_types, acc);
+            break;
         }
     }
-    if (ENERGY) {
-        // every row of a wavefront belongs to this block's group: one sum and
-        // one atomic per kind for the whole wavefront
-        ae0 = warp_sum(ae0, 64);
-        ae1 = warp_sum(ae1, 64);
-        ae2 = warp_sum(ae2, 64);
-        ae3 = warp_sum(ae3, 64);
-        if ((threadIdx.x & 63u) == 0) {
-            const long long v[4] = {ae0, ae1, ae2, ae3};
-            // kinds 4.. are alone in their groups and leave their energy in slot 0
-#pragma unroll
-            for (int k = 0; k < kPairKinds; ++k)
-                if ((kinds >> k) & 1)
-                    atomicAdd(reinterpret_cast<unsigned long long*>(&energy[G.sys * 32 + G.egroup[k]]),
-                              static_cast<unsigned long long>(v[k < 4 ? k : 0]));
-        }
-    } else {
-        const unsigned long long off = acc.nadd * kFixMagicBits;
-        long long ax = static_cast<long long>(acc.ux - off);
-        long long ay = static_cast<long long>(acc.uy - off);
-        long long az = static_cast<long long>(acc.uz - off);
-        ax = warp_sum(ax, TEAM);
-        ay = warp_sum(ay, TEAM);
-        az = warp_sum(az, TEAM);
-        if (lane == 0 && bead_i >= 0) {
-            atomicAdd(reinterpret_cast<unsigned long long*>(&out.fx[bead_i]), static_cast<unsigned long long>(ax));
-            atomicAdd(reinterpret_cast<unsigned long long*>(&out.fy[bead_i]), static_cast<unsigned long long>(ay));
-            atomicAdd(reinterpret_cast<unsigned long long*>(&out.fz[bead_i]), static_cast<unsigned long long>(az));
-        }
+    const unsigned long long off = acc.nadd * kFixMagicBits;
+    long long ax = static_cast<long long>(acc.ux - off);
+    long long ay = static_cast<long long>(acc.uy - off);
+    long long az = static_cast<long long>(acc.uz - off);
+    ax = warp_sum(ax, TEAM);
+    ay = warp_sum(ay, TEAM);
+    az = warp_sum(az, TEAM);
+    if (lane == 0 && bead_i >= 0) {
+        atomicAdd(reinterpret_cast<unsigned long long*>(&out.fx[bead_i]), static_cast<unsigned long long>(ax));
+        atomicAdd(reinterpret_cast<unsigned long long*>(&out.fy[bead_i]), static_cast<unsigned long long>(ay));
+        atomicAdd(reinterpret_cast<unsigned long long*>(&out.fz[bead_i]), static_cast<unsigned long long>(az));
     }
     if (acc.bad) atomicOr(&err[G.sys], kErrNumeric);
     }  // block table
@@ -2049,6 +2002,90 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
         __syncthreads();
         if (threadIdx.x == 0) stamp[2 * blockIdx.x + 1] = static_cast<unsigned long long>(wall_clock64());
     }
+}
+
+// Energy pass: FP64 terms of each pair once (row < column) over the outer
+// list, a team of TEAM lanes per row of the force pass's block table.  A
+// workgroup sums the rows it walks of one group and adds the sums to its copy
+// of the energy words when the group changes: all sums land on a few words,
+// and atomics on one word are served one at a time (~12 ns each).  With one
+// atomic per table entry, wavefront and kind on a single copy the pass took
+// 116 us on the 14,000-bead slab (9,000 in a row on a word), and forces and
+// energies of a frame 736 us; with the kinetic sums spread the same way the
+// frame takes 519 us.
+template <int TEAM>
+__global__ __launch_bounds__(kPairBlock) void k_pair_energy(
+    const DevPairGroup* __restrict__ groups, const int2* __restrict__ blocks, const PairRec* __restrict__ rec,
+    const int* __restrict__ row_start, const int* __restrict__ row_count, const int* __restrict__ col,
+    const double* __restrict__ types_d, long long* __restrict__ energy, int ecopies, int estride, uint32_t gmask,
+    int* __restrict__ err, int nblocks) {
+    energy += static_cast<size_t>(blockIdx.x & (ecopies - 1)) * estride;
+    long long ae0 = 0, ae1 = 0, ae2 = 0, ae3 = 0;
+    int egroup = -1;
+    const auto flush = [&]() {
+        if (egroup < 0) return;   // uniform over the workgroup
+        const DevPairGroup& Q = groups[egroup];
+        const int k = group_kinds(Q, gmask);
+        // every row summed since the last flush belongs to this group
+        const long long v[4] = {warp_sum(ae0, 64), warp_sum(ae1, 64), warp_sum(ae2, 64), warp_sum(ae3, 64)};
+        if ((threadIdx.x & 63u) == 0) {
+            // kinds 4.. are alone in their groups and leave their energy in slot 0
+#pragma unroll
+            for (int b = 0; b < kPairKinds; ++b)
+                if ((k >> b) & 1)
+                    atomicAdd(reinterpret_cast<unsigned long long*>(&energy[Q.sys * 32 + Q.egroup[b]]),
+                              static_cast<unsigned long long>(v[b < 4 ? b : 0]));
+        }
+        ae0 = ae1 = ae2 = ae3 = 0;
+    };
+    for (int bi = static_cast<int>(blockIdx.x); bi < nblocks; bi += static_cast<int>(gridDim.x)) {
+        const int2 bt = blocks[bi];
+        if (bt.x < 0) continue;   // bonded terms: k_bonded
+        const DevPairGroup& G = groups[bt.x];
+        const int kinds = group_kinds(G, gmask);
+        if (bt.x != egroup) {
+            flush();
+            egroup = bt.x;
+        }
+        const int lane = threadIdx.x % TEAM;
+        const int row = bt.y + threadIdx.x / TEAM;
+        if (row >= G.member_begin + G.member_count || !kinds) continue;
+        const bool periodic = G.periodic != 0;
+        const PairK<double> Kd = pair_constants<double>(G);
+        const PairRec ri = rec[row];
+        const int beg = row_start[row], cnt = row_count[row];
+        const double* tdi = types_d + static_cast<size_t>(G.type_begin + (ri.type & 0xFFFF)) * kTypeStride;
+        const int4* col4 = reinterpret_cast<const int4*>(col + beg);
+        int bad = 0;
+        for (int k = lane; 4 * k < cnt; k += TEAM) {
+            const int4 c4 = col4[k];
+            const int cs[4] = {c4.x, c4.y, c4.z, c4.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int s = cs[u];
+                if (s < 0 || row >= s) continue;
+                const PairRec rj = rec[s];
+                double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
+                if (periodic) {
+                    dx = min_image(dx, G.box[0], G.inv_box[0]);
+                    dy = min_image(dy, G.box[1], G.inv_box[1]);
+                    dz = min_image(dz, G.box[2], G.inv_box[2]);
+                }
+                const double r2 = dist2(dx, dy, dz);
+                if (!(r2 < G.rc2)) continue;
+                double f;
+                double e[4] = {0, 0, 0, 0};
+                const double* tdj = types_d + static_cast<size_t>(G.type_begin + (rj.type & 0xFFFF)) * kTypeStride;
+                pair_eval<double>(kinds, Kd, nullptr, nullptr, tdi, tdj, r2, &f, e);
+                ae0 += to_fix_d(e[0], bad);
+                ae1 += to_fix_d(e[1], bad);
+                ae2 += to_fix_d(e[2], bad);
+                ae3 += to_fix_d(e[3], bad);
+            }
+        }
+        if (bad) atomicOr(&err[G.sys], kErrNumeric);
+    }
+    flush();
 }
 
 // ------------------------------------------------------------ resident step
@@ -2602,17 +2639,34 @@ __global__ __launch_bounds__(256) void k_reduce_stamps(const unsigned long long*
 }
 
 // ------------------------------------------------------------- energies
+// One atomic per wavefront and system, into the workgroup's copy of the energy
+// words: with one per bead, all on one word, the 14,000-bead slab took 169 us.
 __global__ void k_kinetic(int nb, const int* __restrict__ sys_of, const double* __restrict__ mass,
                           const double* __restrict__ vx, const double* __restrict__ vy,
-                          const double* __restrict__ vz, long long* __restrict__ ke,
+                          const double* __restrict__ vz, long long* __restrict__ ke, int ecopies, int estride,
                           int* __restrict__ err) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nb) return;
-    const double e = 0.5 * mass[b] * (vx[b] * vx[b] + vy[b] * vy[b] + vz[b] * vz[b]);
-    int bad = 0;
-    const long long q = to_fix_d(e, bad);
-    atomicAdd(reinterpret_cast<unsigned long long*>(&ke[sys_of[b]]), static_cast<unsigned long long>(q));
-    if (bad) atomicOr(&err[sys_of[b]], kErrNumeric);
+    ke += static_cast<size_t>(blockIdx.x & (ecopies - 1)) * estride;
+    long long q = 0;
+    int key = -1;
+    if (b < nb) {
+        const double e = 0.5 * mass[b] * (vx[b] * vx[b] + vy[b] * vy[b] + vz[b] * vz[b]);
+        int bad = 0;
+        q = to_fix_d(e, bad);
+        key = sys_of[b];
+        if (bad) atomicOr(&err[key], kErrNumeric);
+    }
+    wave_add_energy(ke, key, q);
+}
+
+// Sums the copies of the energy words (energies, then kinetic energies of
+// every system) into copy 0.  Whole-number sums: any order, the same bits.
+__global__ void k_energy_reduce(long long* __restrict__ energy, int ecopies, int estride, int n) {
+    const int w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= n) return;
+    unsigned long long v = 0;
+    for (int c = 0; c < ecopies; ++c) v += static_cast<unsigned long long>(energy[static_cast<size_t>(c) * estride + w]);
+    energy[w] = static_cast<long long>(v);
 }
 
 // Lists the interacting pairs (r < cutoff) of one pair group as bead pairs
@@ -2782,29 +2836,29 @@ void launch_bonded(const DevPtrs& d, hipStream_t st, bool energy, const ForceBuf
     ForceOut o{f.fx, f.fy, f.fz};
     if (energy)
         k_bonded<true><<<nblk(d.nt, 256), 256, 0, st>>>(d.nt, d.terms, d.sys, d.sys_of, d.px, d.py, d.pz,
-                                                        d.fla, d.fld, o, d.energy, groups, d.err);
+                                                        d.fla, d.fld, o, d.energy, d.ecopies, d.estride,
+                                                        groups, d.err);
     else
         k_bonded<false><<<nblk(d.nt, 256), 256, 0, st>>>(d.nt, d.terms, d.sys, d.sys_of, d.px, d.py, d.pz,
-                                                         d.fla, d.fld, o, d.energy, groups, d.err);
+                                                         d.fla, d.fld, o, d.energy, d.ecopies, d.estride,
+                                                         groups, d.err);
 }
 
-template <bool E>
 static void pair_dispatch(const DevPtrs& d, hipStream_t st, const ForceBuf& f, uint32_t groups,
                           const int* count, const int* col, unsigned long long* stamp) {
-    const size_t lds = E ? 0 : static_cast<size_t>(d.max_types) * kTypeStride * sizeof(float);
+    const size_t lds = static_cast<size_t>(d.max_types) * kTypeStride * sizeof(float);
     const BondedArgs bd{d.nt, d.terms, d.sys, d.sys_of, d.px, d.py, d.pz, d.fla, d.fld};
     const dim3 grid(std::min(d.n_pair_blocks, d.pair_grid)), block(kPairBlock);
-#define OCM_PAIR(T, U)                                                                                    \
-    if (d.xcd_sliced)                                                                                     \
-        k_pair<E, T, true, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, count, \
-                                                        col, d.types_f, d.types_d, f, d.energy, groups,   \
-                                                        d.err, d.n_pair_blocks, d.nm, stamp, bd);         \
-    else                                                                                                  \
-        k_pair<E, T, false, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, count, \
-                                                         col, d.types_f, d.types_d, f, d.energy, groups,  \
-                                                         d.err, d.n_pair_blocks, d.nm, stamp, bd)
-    // the energy pass has its own loop and always runs the 4-entry instance
-    if (!E && d.pair_u == 2) {
+#define OCM_PAIR(T, U)                                                                                       \
+    if (d.xcd_sliced)                                                                                        \
+        k_pair<T, true, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, count, col, \
+                                                     d.types_f, f, groups, d.err, d.n_pair_blocks, d.nm,     \
+                                                     stamp, bd);                                             \
+    else                                                                                                     \
+        k_pair<T, false, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, count, col, \
+                                                      d.types_f, f, groups, d.err, d.n_pair_blocks, d.nm,    \
+                                                      stamp, bd)
+    if (d.pair_u == 2) {
         switch (d.team) {
         case 8: OCM_PAIR(8, 2); break;
         case 32: OCM_PAIR(32, 2); break;
@@ -2820,6 +2874,26 @@ static void pair_dispatch(const DevPtrs& d, hipStream_t st, const ForceBuf& f, u
         }
     }
 #undef OCM_PAIR
+}
+
+// Energy pass over the outer list (few enough workgroups that their final
+// sums stay few).
+constexpr int kEnergyGrid = 2048;
+
+static void energy_dispatch(const DevPtrs& d, hipStream_t st, uint32_t groups) {
+    const dim3 grid(std::min(d.n_pair_blocks, kEnergyGrid)), block(kPairBlock);
+#define OCM_ENERGY(T)                                                                                       \
+    k_pair_energy<T><<<grid, block, 0, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, d.row_count, d.col, \
+                                             d.types_d, d.energy, d.ecopies, d.estride, groups, d.err,       \
+                                             d.n_pair_blocks)
+    switch (d.team) {
+    case 4: OCM_ENERGY(4); break;
+    case 8: OCM_ENERGY(8); break;
+    case 32: OCM_ENERGY(32); break;
+    case 64: OCM_ENERGY(64); break;
+    default: OCM_ENERGY(16); break;
+    }
+#undef OCM_ENERGY
 }
 
 void launch_prune(const DevPtrs& d, hipStream_t st) {
@@ -2846,12 +2920,12 @@ void launch_pair(const DevPtrs& d, hipStream_t st, bool energy, const ForceBuf& 
     // outer list is read and nothing is written
     if (!d.col_in || energy || (list == kListPrune && groups != 0xFFFFFFFFu)) list = kListOuter;
     if (energy) {
-        pair_dispatch<true>(d, st, f, groups, d.row_count, d.col, stamp);
+        energy_dispatch(d, st, groups);
         return;
     }
     if (list == kListPrune) launch_prune(d, st);   // then the force pass reads the fresh inner list
-    if (list == kListOuter) pair_dispatch<false>(d, st, f, groups, d.row_count, d.col, stamp);
-    else pair_dispatch<false>(d, st, f, groups, d.row_count_in, d.col_in, stamp);
+    if (list == kListOuter) pair_dispatch(d, st, f, groups, d.row_count, d.col, stamp);
+    else pair_dispatch(d, st, f, groups, d.row_count_in, d.col_in, stamp);
 }
 
 int pair_grid_size(const DevPtrs& d) { return std::min(d.n_pair_blocks, d.pair_grid); }
@@ -2888,12 +2962,19 @@ void launch_reduce_stamps(hipStream_t st, const unsigned long long* stamp, int n
 }
 
 void launch_zero_energy(const DevPtrs& d, hipStream_t st) {
-    k_fill_i64<<<nblk(d.nsys * 32, 256), 256, 0, st>>>(d.energy, 0, d.nsys * 32);
-    k_fill_i64<<<nblk(d.nsys, 256), 256, 0, st>>>(d.ke, 0, d.nsys);
+    const int n = d.ecopies * d.estride;
+    k_fill_i64<<<nblk(n, 256), 256, 0, st>>>(d.energy, 0, n);
 }
 
 void launch_kinetic(const DevPtrs& d, hipStream_t st) {
-    k_kinetic<<<nblk(d.nb, 256), 256, 0, st>>>(d.nb, d.sys_of, d.mass, d.vx, d.vy, d.vz, d.ke, d.err);
+    k_kinetic<<<nblk(d.nb, 256), 256, 0, st>>>(d.nb, d.sys_of, d.mass, d.vx, d.vy, d.vz, d.energy + d.nsys * 32,
+                                               d.ecopies, d.estride, d.err);
+}
+
+void launch_energy_reduce(const DevPtrs& d, hipStream_t st) {
+    if (d.ecopies == 1) return;
+    const int n = d.nsys * 33;
+    k_energy_reduce<<<nblk(n, 256), 256, 0, st>>>(d.energy, d.ecopies, d.estride, n);
 }
 
 void launch_neighbor_dump(const DevPtrs& d, hipStream_t st, int group, long long cap, int members,

@@ -87,8 +87,11 @@ struct DevPtrs {
     BTerm* res_terms = nullptr;
     float* res_rows = nullptr;
     uint32_t* res_list = nullptr;
-    long long* energy = nullptr;   // nsys * 32 fixed point
-    long long* ke = nullptr;       // nsys fixed point
+    // fixed-point energies: ecopies (a power of two) copies of estride words,
+    // each the nsys * 32 group energies, then the nsys kinetic energies;
+    // workgroups add to different copies, launch_energy_reduce sums them into copy 0
+    long long* energy = nullptr;
+    int ecopies = 1, estride = 0;
     int* dump_count = nullptr;
 };
 
@@ -136,6 +139,7 @@ void launch_reduce_stamps(hipStream_t st, const unsigned long long* stamp, int n
                           unsigned long long* out);
 void launch_zero_energy(const DevPtrs& d, hipStream_t st);
 void launch_kinetic(const DevPtrs& d, hipStream_t st);
+void launch_energy_reduce(const DevPtrs& d, hipStream_t st);
 // Interacting pairs (r < cutoff, i < j as global bead ids) of one pair group
 // into out (up to cap pairs); *count receives how many there are.
 void launch_neighbor_dump(const DevPtrs& d, hipStream_t st, int group, long long cap, int members,
