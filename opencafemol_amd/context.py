@@ -99,7 +99,7 @@ class Batch:
         arrs = {}
         for key, bit in (("positions", 1), ("velocities", 2), ("forces", 4)):
             if what & bit:
-                arrs[key] = np.zeros((n, 3))
+                arrs[key] = np.empty((n, 3))
                 setattr(st, key, arrs[key].ctypes.data_as(C.POINTER(C.c_double)))
         check(self.lib.ocm_batch_get_state(self.h, s, what, groups, C.byref(st)))
         out.update(arrs)

@@ -635,12 +635,22 @@ void Engine::pack() {
     bstate_ = dalloc<double>(3 * static_cast<size_t>(n3) + 2);
     {
         // pinned, device-mapped and coherent: the chunk's last kernel writes
-        // the status words straight into it
+        // the status words straight into it; behind them the head of a state
+        // read and the staging of its arrays.  Up to 1 MiB is staged (14,000
+        // beads' positions and velocities): past that the host's copy out of
+        // the staging costs more than the runtime's own copy to the caller.
         void* h = nullptr;
-        check_hip(hipHostMalloc(&h, sizeof(int) * (1 + static_cast<size_t>(nsys)),
-                                hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
+        size_t max_n = 0;
+        for (const HostSystem& H : sys_) max_n = std::max<size_t>(max_n, H.n);
+        const size_t status_bytes = (sizeof(int) * (1 + static_cast<size_t>(nsys)) + 63) & ~static_cast<size_t>(63);
+        const size_t head_bytes = (sizeof(long long) * kStateHead + 63) & ~static_cast<size_t>(63);
+        stage_doubles_ = std::min<size_t>(9 * max_n, (1u << 20) / sizeof(double));
+        const size_t bytes = status_bytes + head_bytes + stage_doubles_ * sizeof(double);
+        check_hip(hipHostMalloc(&h, bytes, hipHostMallocMapped | hipHostMallocCoherent), "hipHostMalloc");
         status_host_ = static_cast<int*>(h);
-        std::memset(status_host_, 0, sizeof(int) * (1 + static_cast<size_t>(nsys)));
+        head_host_ = reinterpret_cast<long long*>(static_cast<char*>(h) + status_bytes);
+        stage_host_ = reinterpret_cast<double*>(static_cast<char*>(h) + status_bytes + head_bytes);
+        std::memset(h, 0, status_bytes + head_bytes);
     }
     d_.sys = dalloc<DevSys>(nsys);
     upload(d_.sys, dsys);
@@ -1029,6 +1039,7 @@ void Engine::collect_timing() {
 
 void Engine::sync() {
     check_hip(hipStreamSynchronize(stream_), "hipStreamSynchronize");
+    stage_busy_ = false;
     if (timing_) collect_timing();
 }
 
@@ -1171,31 +1182,26 @@ void Engine::grow_rows() {
 
 // Device error words are cleared after every read.  Flags raised by a force
 // evaluation outside a chunk (the one that starts stepping) are carried on the
-// host and reported with the next accepted chunk.
+// host and reported with the next accepted chunk.  Enqueued status words must
+// have been waited for.
 void Engine::carry_errors() {
-    sync();
-    std::vector<int> err(d_.nsys);
-    check_hip(hipMemcpy(err.data(), d_.err, sizeof(int) * d_.nsys, hipMemcpyDeviceToHost), "err");
-    for (int s = 0; s < d_.nsys; ++s) err_carry_[s] |= err[s] & kErrNumeric;
-    check_hip(hipMemsetAsync(d_.err, 0, sizeof(int) * d_.nsys, stream_), "memset");
+    for (int s = 0; s < d_.nsys; ++s) err_carry_[s] |= status_host_[1 + s] & kErrNumeric;
 }
 
 void Engine::ensure_forces() {
     const TraceRange trace("ocm.forces");
     if (!forces_dirty_) return;
     for (int attempt = 0; attempt < 8; ++attempt) {
-        check_hip(hipMemsetAsync(d_.flags, 0, sizeof(int), stream_), "memset");
-        check_hip(hipMemsetAsync(d_.err, 0, sizeof(int) * d_.nsys, stream_), "memset");
-        launch_zero_forces(d_, d_.f, stream_);
+        launch_eval_begin(d_, d_.f, stream_);
         enqueue_forces(d_.f, true, 0xFFFFFFFFu);
+        launch_status_out(d_, stream_, status_host_);
         sync();
-        int flags = 0;
-        check_hip(hipMemcpy(&flags, d_.flags, sizeof(int), hipMemcpyDeviceToHost), "flags");
-        if (flags & kFlagListOverflow) {
+        if (status_host_[0] & kFlagListOverflow) {
             grow_rows();
             continue;
         }
         forces_dirty_ = false;
+        list_current_ = true;
         // built and pruned outside a chunk (the prune positions are not
         // recorded there): the next chunk starts with a rebuild
         stale_lists();
@@ -1203,6 +1209,8 @@ void Engine::ensure_forces() {
             autotune_team();   // clears the flags its scratch launches raised
             launch_zero_forces(d_, d_.f, stream_);
             enqueue_forces(d_.f, false, 0xFFFFFFFFu);   // again, with the tuned launch shape
+            launch_status_out(d_, stream_, status_host_);
+            sync();
         }
         carry_errors();
         return;
@@ -1431,8 +1439,7 @@ int Engine::step_resident(long long n) {
     long long remaining = n;
     while (remaining > 0) {
         const int k = static_cast<int>(std::min<long long>(remaining, kResChunk));
-        launch_resident(d_, stream_, k);
-        launch_status_out(d_, stream_, status_host_);
+        launch_resident(d_, stream_, k, status_host_);
         sync();
         const int* err = status_host_ + 1;
         for (int s = 0; s < d_.nsys; ++s) {
@@ -1455,6 +1462,7 @@ int Engine::step(long long n) {
     if (n < 0) invalid("negative step count");
     if (n == 0) return OCM_OK;
     ensure_forces();
+    list_current_ = false;
     if (d_.res_n > 0) return step_resident(n);
     int status = OCM_OK;
     long long remaining = n;
@@ -1518,6 +1526,7 @@ int Engine::minimize(double tol, int max_iter) {
     auto evaluate = [&](const std::vector<double>& x, std::vector<double>& g) {
         check_hip(hipMemcpy(d_.px, x.data(), n3 * sizeof(double), hipMemcpyHostToDevice), "positions");
         forces_dirty_ = true;
+        list_current_ = false;
         ensure_forces();
         check_hip(hipMemcpy(fbuf.data(), d_.f.fx, n3 * sizeof(long long), hipMemcpyDeviceToHost), "forces");
         const std::vector<double> pe = potentials();
@@ -1614,6 +1623,7 @@ int Engine::minimize(double tol, int max_iter) {
     check_hip(hipMemset(d_.err, 0, sizeof(int) * d_.nsys), "memset");
     std::fill(err_carry_.begin(), err_carry_.end(), 0);
     forces_dirty_ = true;
+    list_current_ = false;
     return it;
 }
 
@@ -1639,30 +1649,33 @@ void Engine::set_steps_done(int s, long long steps_done) {
 }
 
 // ------------------------------------------------------------ state I/O
-void Engine::set_positions(int s, const double* xyz) {
-    const HostSystem& H = sys_.at(s);
-    std::vector<double> x(H.n), y(H.n), z(H.n);
-    for (int i = 0; i < H.n; ++i) {
-        x[i] = xyz[3 * i]; y[i] = xyz[3 * i + 1]; z[i] = xyz[3 * i + 2];
-        if (!std::isfinite(x[i]) || !std::isfinite(y[i]) || !std::isfinite(z[i])) invalid("position is not finite");
+// xyz rows of system s into a bead array (x, y and z blocks at dst).
+void Engine::put_rows(int s, const double* xyz, double* dst) {
+    const size_t words = 3 * static_cast<size_t>(sys_.at(s).n);
+    const double* in = stage_host_;
+    if (words <= stage_doubles_) {
+        if (stage_busy_) sync();   // an earlier upload still reads the staging
+        std::memcpy(stage_host_, xyz, words * sizeof(double));
+        stage_busy_ = true;
+    } else {
+        sync();   // nothing on the stream uses the device buffer
+        check_hip(hipMemcpy(bstate_, xyz, words * sizeof(double), hipMemcpyHostToDevice), "state upload");
+        in = bstate_;
     }
-    const size_t off = bead_begin_[s];
-    check_hip(hipMemcpy(d_.px + off, x.data(), H.n * sizeof(double), hipMemcpyHostToDevice), "positions");
-    check_hip(hipMemcpy(d_.py + off, y.data(), H.n * sizeof(double), hipMemcpyHostToDevice), "positions");
-    check_hip(hipMemcpy(d_.pz + off, z.data(), H.n * sizeof(double), hipMemcpyHostToDevice), "positions");
+    launch_state_in(d_, stream_, bead_begin_[s], sys_[s].n, in, dst);
+}
+
+void Engine::set_positions(int s, const double* xyz) {
+    const size_t words = 3 * static_cast<size_t>(sys_.at(s).n);
+    for (size_t i = 0; i < words; ++i)
+        if (!std::isfinite(xyz[i])) invalid("position is not finite");
+    put_rows(s, xyz, d_.px);
     forces_dirty_ = true;
+    list_current_ = false;
     sys_status_[s] = OCM_OK;
 }
 
-void Engine::set_velocities(int s, const double* xyz) {
-    const HostSystem& H = sys_.at(s);
-    std::vector<double> x(H.n), y(H.n), z(H.n);
-    for (int i = 0; i < H.n; ++i) { x[i] = xyz[3 * i]; y[i] = xyz[3 * i + 1]; z[i] = xyz[3 * i + 2]; }
-    const size_t off = bead_begin_[s];
-    check_hip(hipMemcpy(d_.vx + off, x.data(), H.n * sizeof(double), hipMemcpyHostToDevice), "velocities");
-    check_hip(hipMemcpy(d_.vy + off, y.data(), H.n * sizeof(double), hipMemcpyHostToDevice), "velocities");
-    check_hip(hipMemcpy(d_.vz + off, z.data(), H.n * sizeof(double), hipMemcpyHostToDevice), "velocities");
-}
+void Engine::set_velocities(int s, const double* xyz) { put_rows(s, xyz, d_.vx); }
 
 void Engine::set_velocities_to_temperature(int s, double T, uint64_t seed) {
     if (!(T >= 0)) invalid("temperature must be >= 0");
@@ -1671,24 +1684,18 @@ void Engine::set_velocities_to_temperature(int s, double T, uint64_t seed) {
     sync();
 }
 
-static void to_host3(const double* dx, const double* dy, const double* dz, int n, double* out) {
-    std::vector<double> x(n), y(n), z(n);
-    (void)hipMemcpy(x.data(), dx, n * sizeof(double), hipMemcpyDeviceToHost);
-    (void)hipMemcpy(y.data(), dy, n * sizeof(double), hipMemcpyDeviceToHost);
-    (void)hipMemcpy(z.data(), dz, n * sizeof(double), hipMemcpyDeviceToHost);
-    for (int i = 0; i < n; ++i) { out[3 * i] = x[i]; out[3 * i + 1] = y[i]; out[3 * i + 2] = z[i]; }
-}
-
 void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
     const TraceRange trace("ocm.get_state");
     const HostSystem& H = sys_.at(s);
-    const size_t off = bead_begin_[s];
-    sync();
-    if ((what & OCM_STATE_POSITIONS) && out->positions) to_host3(d_.px + off, d_.py + off, d_.pz + off, H.n, out->positions);
-    if ((what & OCM_STATE_VELOCITIES) && out->velocities) to_host3(d_.vx + off, d_.vy + off, d_.vz + off, H.n, out->velocities);
-    long long gs[2] = {0, 0};
-    check_hip(hipMemcpy(gs, d_.gstep, sizeof(gs), hipMemcpyDeviceToHost), "gstep");
-    out->step = gs[0] - sys_step_origin_[s];
+    StateOut o;
+    o.sys = s; o.nsys = d_.nsys; o.off = bead_begin_[s]; o.n = H.n; o.nb = d_.nb;
+    o.gstep = d_.gstep; o.flags = d_.flags; o.err = d_.err;
+    o.head = head_host_;
+    // where each array's rows go, in the order k_state_out writes them
+    double* dst[3] = {};
+    int nrows = 0;
+    if ((what & OCM_STATE_POSITIONS) && out->positions) { o.pos = d_.px; dst[nrows++] = out->positions; }
+    if ((what & OCM_STATE_VELOCITIES) && out->velocities) { o.vel = d_.vx; dst[nrows++] = out->velocities; }
     if ((what & OCM_STATE_FORCES) && out->forces) {
         const uint32_t present = sys_group_mask_[s];
         ForceBuf src = d_.f;
@@ -1698,46 +1705,55 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
             enqueue_forces(d_.f2, false, groups);
             src = d_.f2;
         }
-        sync();
-        // a read of forces raises no step error (the full evaluation's flags are carried)
-        check_hip(hipMemsetAsync(d_.err, 0, sizeof(int) * d_.nsys, stream_), "memset");
-        std::vector<long long> fx(H.n), fy(H.n), fz(H.n);
-        check_hip(hipMemcpy(fx.data(), src.fx + off, H.n * sizeof(long long), hipMemcpyDeviceToHost), "forces");
-        check_hip(hipMemcpy(fy.data(), src.fy + off, H.n * sizeof(long long), hipMemcpyDeviceToHost), "forces");
-        check_hip(hipMemcpy(fz.data(), src.fz + off, H.n * sizeof(long long), hipMemcpyDeviceToHost), "forces");
-        for (int i = 0; i < H.n; ++i) {
-            out->forces[3 * i] = fx[i] * kFixInv;
-            out->forces[3 * i + 1] = fy[i] * kFixInv;
-            out->forces[3 * i + 2] = fz[i] * kFixInv;
-        }
+        o.frc = src.fx;
+        o.clear_err = 1;   // the full evaluation's flags are carried
+        dst[nrows++] = out->forces;
     }
     if (what & OCM_STATE_ENERGY) {
         launch_zero_energy(d_, stream_);
-        if (d_.nm > 0) { launch_rebuild(d_, stream_); ++rebuilds_; stale_lists(); }
+        if (d_.nm > 0 && (!list_current_ || lists_stale_)) {
+            launch_rebuild(d_, stream_);
+            ++rebuilds_;
+            lists_stale_ = false;
+            list_current_ = true;
+            stale_lists();
+        }
         launch_bonded(d_, stream_, true, d_.f2, groups);
         launch_pair(d_, stream_, true, d_.f2, groups);
         launch_kinetic(d_, stream_);
-        launch_energy_reduce(d_, stream_);
-        sync();
-        check_hip(hipMemsetAsync(d_.err, 0, sizeof(int) * d_.nsys, stream_), "memset");   // energies raise no step error
-        int flags = 0;
-        check_hip(hipMemcpy(&flags, d_.flags, sizeof(int), hipMemcpyDeviceToHost), "flags");
-        if (flags & kFlagListOverflow) {
-            grow_rows();
-            check_hip(hipMemset(d_.flags, 0, sizeof(int)), "memset");
-            get_state(s, OCM_STATE_ENERGY, groups, out);
-            return;
-        }
-        std::vector<long long> e(32);
-        long long ke = 0;
-        check_hip(hipMemcpy(e.data(), d_.energy + static_cast<size_t>(s) * 32, 32 * sizeof(long long), hipMemcpyDeviceToHost), "energy");
-        check_hip(hipMemcpy(&ke, d_.energy + static_cast<size_t>(d_.nsys) * 32 + s, sizeof(long long), hipMemcpyDeviceToHost), "ke");
+        o.clear_err = 1;
+        o.energy = d_.energy;
+        o.ecopies = d_.ecopies;
+        o.estride = d_.estride;
+    }
+    const size_t words = 3 * static_cast<size_t>(H.n) * nrows;
+    const bool staged = words <= stage_doubles_;
+    if (!staged) sync();   // nothing on the stream uses the device buffer
+    o.data = staged ? stage_host_ : bstate_;
+    if (nrows == 0) o.n = 0;
+    launch_state_out(stream_, o);
+    sync();
+    if ((what & OCM_STATE_ENERGY) && (head_host_[1] & kFlagListOverflow)) {
+        // the rebuild found a row longer than its slots
+        grow_rows();
+        list_current_ = false;
+        check_hip(hipMemset(d_.flags, 0, sizeof(int)), "memset");
+        get_state(s, what, groups, out);
+        return;
+    }
+    out->step = head_host_[0] - sys_step_origin_[s];
+    for (int k = 0; k < nrows; ++k) {
+        const size_t bytes = 3 * static_cast<size_t>(H.n) * sizeof(double);
+        if (staged) std::memcpy(dst[k], stage_host_ + 3 * static_cast<size_t>(H.n) * k, bytes);
+        else check_hip(hipMemcpy(dst[k], bstate_ + 3 * static_cast<size_t>(H.n) * k, bytes, hipMemcpyDeviceToHost), "state");
+    }
+    if (what & OCM_STATE_ENERGY) {
         out->potential_energy = 0;
         for (int g = 0; g < 32; ++g) {
-            out->energy_by_group[g] = e[g] * kFixInv;
+            out->energy_by_group[g] = head_host_[2 + g] * kFixInv;
             if ((groups >> g) & 1u) out->potential_energy += out->energy_by_group[g];
         }
-        out->kinetic_energy = ke * kFixInv;
+        out->kinetic_energy = head_host_[34] * kFixInv;
     }
 }
 
@@ -1753,6 +1769,7 @@ int Engine::pair_group_of(int s, int force_index) const {
 // Rebuilds the outer list at the current positions; returns the flag word.
 int Engine::rebuild_now() {
     lists_stale_ = false;
+    list_current_ = false;
     launch_fill_i32(stream_, d_.flags, 0, 1);
     launch_rebuild(d_, stream_);
     ++rebuilds_;

@@ -125,6 +125,7 @@ private:
     int pair_group_of(int s, int force_index) const;
     int rebuild_now();
     void carry_errors();
+    void put_rows(int s, const double* xyz, double* dst);
     void enqueue_forces(const ForceBuf& f, bool rebuild, uint32_t groups);
     // List schedule of one chunk: which steps rebuild the outer list and which
     // prune the inner one, from the list ages carried in from earlier chunks.
@@ -209,6 +210,15 @@ private:
     // pinned host words the chunk's last kernel writes: the batch flag word,
     // then one error word per system (cleared on the device as they are copied)
     int* status_host_ = nullptr;
+    // in the same pinned allocation: the head of a state read, and staging for
+    // the bead arrays of systems up to stage_doubles_ (larger ones go through
+    // bstate_, which only a running chunk uses)
+    long long* head_host_ = nullptr;
+    double* stage_host_ = nullptr;
+    size_t stage_doubles_ = 0;
+    bool stage_busy_ = false;   // a kernel not yet waited for reads the staging
+    // the outer list was built at the current positions
+    bool list_current_ = false;
     unsigned long long* stamp_host_ = nullptr;   // 2 words per step of a chunk (timing mode 2)
 
     // ages of the lists, carried from chunk to chunk: steps since the outer

@@ -117,15 +117,74 @@ __global__ void k_snapshot(int n3, const double* __restrict__ pos, const double*
 
 // Last kernel of a chunk: copies the flag word and the per-system error
 // words into pinned host memory (host[0] flags, host[1 + s] system s) and
-// clears the error words for the next chunk.
+// clears the error words for the next chunk.  advance > 0 (resident chunks):
+// both step slots move on by that many steps.
 __global__ void k_status_out(int nsys, const int* __restrict__ flags, int* __restrict__ err,
-                             int* __restrict__ host) {
+                             int* __restrict__ host, long long* gstep, int advance) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t == 0) host[0] = *flags;
+    if (t == 0) {
+        host[0] = *flags;
+        if (advance > 0) {
+            const long long s = gstep[0] + advance;
+            gstep[0] = s;
+            gstep[1] = s;
+        }
+    }
     for (int s = t; s < nsys; s += gridDim.x * blockDim.x) {
         host[1 + s] = err[s];
         err[s] = 0;
     }
+}
+
+// Start of a force evaluation outside a chunk: force words, flag word and
+// error words to zero in one launch.
+__global__ void k_eval_begin(int n3, long long* __restrict__ f, int* __restrict__ flags, int* __restrict__ err,
+                             int nsys) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) *flags = 0;
+    for (int s = t; s < nsys; s += gridDim.x * blockDim.x) err[s] = 0;
+    if (t < n3) f[t] = 0;
+}
+
+// One system's state for the caller: head (pinned host memory: step slot, flag
+// word, the 32 group energies and the kinetic energy, summed over the copies
+// of the energy words) and the bead arrays of `what` as xyz rows, into pinned
+// host memory or a device buffer.  One launch and one wait in place of up to
+// eleven blocking copies and the transposition on the host: the latency of
+// the calls bounds small systems (a 62-bead frame).
+__global__ void k_state_out(StateOut a) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (blockIdx.x == 0) {
+        if (threadIdx.x == 33) a.head[0] = a.gstep[0];
+        if (threadIdx.x == 34) a.head[1] = *a.flags;
+        if (a.energy && threadIdx.x < 33) {
+            const int w = threadIdx.x < 32 ? a.sys * 32 + static_cast<int>(threadIdx.x) : a.nsys * 32 + a.sys;
+            unsigned long long v = 0;
+            for (int c = 0; c < a.ecopies; ++c)
+                v += static_cast<unsigned long long>(a.energy[static_cast<size_t>(c) * a.estride + w]);
+            a.head[2 + threadIdx.x] = static_cast<long long>(v);
+        }
+        // a read of forces or energies raises no step error
+        if (a.clear_err)
+            for (int s = threadIdx.x; s < a.nsys; s += blockDim.x) a.err[s] = 0;
+    }
+    if (t >= 3 * a.n) return;
+    // thread t writes word t of each array's rows: consecutive stores
+    const int b = t / 3, c = t - 3 * b;
+    const size_t src = static_cast<size_t>(c) * a.nb + a.off + b;
+    double* out = a.data;
+    if (a.pos) { out[t] = a.pos[src]; out += 3 * static_cast<size_t>(a.n); }
+    if (a.vel) { out[t] = a.vel[src]; out += 3 * static_cast<size_t>(a.n); }
+    if (a.frc) out[t] = static_cast<double>(a.frc[src]) * kFixInv;
+}
+
+// The reverse for positions or velocities: xyz rows (pinned host memory or a
+// device buffer) into the bead arrays.
+__global__ void k_state_in(int n, int off, int nb, const double* __restrict__ in, double* __restrict__ dst) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3 * n) return;
+    const int b = t / 3, c = t - 3 * b;
+    dst[static_cast<size_t>(c) * nb + off + b] = in[t];
 }
 
 // ---------------------------------------------------- record refresh
@@ -2126,8 +2185,10 @@ struct ResArgs {
     uint32_t* list;
     const FlaTable* fla;
     const FldTable* fld;
-    const long long* gstep;
+    long long* gstep;
     int* err;
+    const int* flags;
+    int* host;                 // pinned status words (k_status_out's), written here when there is one workgroup
     int nsteps;
     int nbs;                   // LDS entries per bead array (>= every system's beads, multiple of 64)
     int term_cap;              // bonded terms staged in LDS per system
@@ -2600,15 +2661,16 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         a.vx[gb] = V[0]; a.vy[gb] = V[1]; a.vz[gb] = V[2];
         a.fx[gb] = F0; a.fy[gb] = F1; a.fz[gb] = F2;
     }
-    if (bad) atomicOr(&a.err[R.sys], kErrNumeric);
-}
-
-// Both step slots advance by n after a resident chunk.
-__global__ void k_gstep_advance(long long* gstep, int n) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const long long s = gstep[0] + n;
-        gstep[0] = s;
-        gstep[1] = s;
+    const int any = __syncthreads_or(bad);
+    if (gridDim.x > 1) {   // k_status_out follows
+        if (tid == 0 && any) atomicOr(&a.err[R.sys], kErrNumeric);
+    } else if (tid == 0) {
+        // the only workgroup: what k_status_out does, one launch less
+        a.host[0] = *a.flags;
+        a.host[1] = a.err[0] | (any ? kErrNumeric : 0);
+        a.err[0] = 0;
+        a.gstep[0] = step0 + a.nsteps;
+        a.gstep[1] = step0 + a.nsteps;
     }
 }
 
@@ -2717,11 +2779,21 @@ __global__ void k_velocity_noise(int nb, int sys, const int* __restrict__ sys_of
 // ------------------------------------------------------------ launchers
 static inline int nblk(long long n, int b) { return static_cast<int>((n + b - 1) / b); }
 
+void launch_eval_begin(const DevPtrs& d, const ForceBuf& f, hipStream_t st) {
+    const int n3 = 3 * d.nb;   // the three force arrays follow each other
+    k_eval_begin<<<nblk(std::max(n3, 1), 256), 256, 0, st>>>(n3, f.fx, d.flags, d.err, d.nsys);
+}
+
 void launch_zero_forces(const DevPtrs& d, const ForceBuf& f, hipStream_t st) {
-    if (d.nb == 0) return;
-    k_fill_i64<<<nblk(d.nb, 256), 256, 0, st>>>(f.fx, 0, d.nb);
-    k_fill_i64<<<nblk(d.nb, 256), 256, 0, st>>>(f.fy, 0, d.nb);
-    k_fill_i64<<<nblk(d.nb, 256), 256, 0, st>>>(f.fz, 0, d.nb);
+    if (d.nb > 0) k_fill_i64<<<nblk(3 * d.nb, 256), 256, 0, st>>>(f.fx, 0, 3 * d.nb);
+}
+
+void launch_state_out(hipStream_t st, const StateOut& a) {
+    k_state_out<<<nblk(std::max(3 * a.n, 1), 256), 256, 0, st>>>(a);
+}
+
+void launch_state_in(const DevPtrs& d, hipStream_t st, int off, int n, const double* in, double* dst) {
+    if (n > 0) k_state_in<<<nblk(3 * n, 256), 256, 0, st>>>(n, off, d.nb, in, dst);
 }
 
 // Small workgroups: a step touches each bead once, so the launch is one
@@ -2742,8 +2814,8 @@ void launch_snapshot(const DevPtrs& d, hipStream_t st, double* snap) {
     k_snapshot<<<nblk(std::max(n3, 1), 256), 256, 0, st>>>(n3, d.px, d.vx, d.f.fx, d.gstep, snap, d.flags);
 }
 
-void launch_status_out(const DevPtrs& d, hipStream_t st, int* host) {
-    k_status_out<<<1, 256, 0, st>>>(d.nsys, d.flags, d.err, host);
+void launch_status_out(const DevPtrs& d, hipStream_t st, int* host, int advance) {
+    k_status_out<<<1, 256, 0, st>>>(d.nsys, d.flags, d.err, host, d.gstep, advance);
 }
 
 void launch_half_kick(const DevPtrs& d, hipStream_t st, int pcur) {
@@ -2941,19 +3013,19 @@ hipError_t resident_prepare(int threads, size_t lds) {
     return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
 }
 
-void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps) {
+void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host) {
     if (d.res_n == 0 || nsteps <= 0) return;
     const ResArgs a{d.res_tab, d.res_grp, d.res_terms, d.res_rows, d.sys, d.groups, d.member_bead, d.member_type,
                     d.local_id, d.inv_m, d.res_hs2, d.px, d.py, d.pz,
-                    d.vx, d.vy, d.vz, d.f.fx, d.f.fy, d.f.fz, d.res_list, d.fla, d.fld, d.gstep, d.err, nsteps,
-                    d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_excl, d.res_ex_cap};
+                    d.vx, d.vy, d.vz, d.f.fx, d.f.fy, d.f.fz, d.res_list, d.fla, d.fld, d.gstep, d.err,
+                    d.flags, host, nsteps, d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_excl, d.res_ex_cap};
     const size_t lds = res_lds_bytes(d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_ex_cap);
     switch (d.res_threads) {
     case 256: k_resident<256><<<d.res_n, 256, lds, st>>>(a); break;
     case 512: k_resident<512><<<d.res_n, 512, lds, st>>>(a); break;
     default: k_resident<1024><<<d.res_n, 1024, lds, st>>>(a); break;
     }
-    k_gstep_advance<<<1, 64, 0, st>>>(d.gstep, nsteps);
+    if (d.res_n > 1) launch_status_out(d, st, host, nsteps);
 }
 
 void launch_reduce_stamps(hipStream_t st, const unsigned long long* stamp, int nlaunch, int nblk,

@@ -100,6 +100,26 @@ constexpr int kPairBlock = 128;
 constexpr double kPruneMargin = 0.1;
 
 void launch_zero_forces(const DevPtrs& d, const ForceBuf& f, hipStream_t st);
+// Force words of f, the flag word and the error words to zero.
+void launch_eval_begin(const DevPtrs& d, const ForceBuf& f, hipStream_t st);
+// One system's state (see k_state_out); null arrays are left out.
+constexpr int kStateHead = 35;   // words of head: step, flags, 32 energies, kinetic
+struct StateOut {
+    int sys = 0, nsys = 0, off = 0, n = 0, nb = 0;
+    const double* pos = nullptr;
+    const double* vel = nullptr;
+    const long long* frc = nullptr;
+    const long long* gstep = nullptr;
+    const int* flags = nullptr;
+    int* err = nullptr;
+    int clear_err = 0;
+    const long long* energy = nullptr;
+    int ecopies = 1, estride = 0;
+    long long* head = nullptr;   // pinned host memory
+    double* data = nullptr;
+};
+void launch_state_out(hipStream_t st, const StateOut& a);
+void launch_state_in(const DevPtrs& d, hipStream_t st, int off, int n, const double* in, double* dst);
 // pack != 0: also refresh the pair records (and check list validity when check != 0).
 // prune: kPruneNone, kPruneWrite (this step's pair pass prunes: record the
 // positions) or kPruneCheck (flag beads that moved more than margin/2 since).
@@ -111,7 +131,7 @@ void launch_half_kick(const DevPtrs& d, hipStream_t st, int pcur);
 // and the two step slots, and the flag word is cleared; host (pinned, 1 + nsys
 // words) receives the flag word and the error words, which are then cleared.
 void launch_snapshot(const DevPtrs& d, hipStream_t st, double* snap);
-void launch_status_out(const DevPtrs& d, hipStream_t st, int* host);
+void launch_status_out(const DevPtrs& d, hipStream_t st, int* host, int advance = 0);
 void launch_pack(const DevPtrs& d, hipStream_t st);
 void launch_rebuild(const DevPtrs& d, hipStream_t st);
 void launch_bonded(const DevPtrs& d, hipStream_t st, bool energy, const ForceBuf& f, uint32_t groups);
@@ -127,9 +147,10 @@ void launch_pair(const DevPtrs& d, hipStream_t st, bool energy, const ForceBuf& 
 void launch_prune(const DevPtrs& d, hipStream_t st);
 int pair_grid_size(const DevPtrs& d);
 // Resident stepping: nsteps steps of every system, each in one workgroup, and
-// both step slots advanced by nsteps.  Forces at the current positions must be
-// in d.f and the velocities synchronized; both hold again afterwards.
-void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps);
+// both step slots advanced by nsteps; host (pinned) receives the status words
+// of launch_status_out.  Forces at the current positions must be in d.f and
+// the velocities synchronized; both hold again afterwards.
+void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host);
 // LDS of one resident workgroup (bead arrays of nbs entries), and the
 // attribute that allows it (gfx950 gives a workgroup up to 160 KB).
 size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap);
