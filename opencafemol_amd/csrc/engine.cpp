@@ -939,7 +939,7 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
 void Engine::build_pair_blocks(int team) {
     d_.team = team;
     const int rpb = kPairBlock / team;
-    std::vector<int2> blocks;
+    std::vector<int4> blocks;
     // Batches of many systems: the pair kernel's workgroups walk the table in
     // 8 contiguous slices, one per XCD (k_pair's SLICED walk), and the table
     // is laid out as 8 slices with the same mix of work: each holds an eighth
@@ -957,16 +957,19 @@ void Engine::build_pair_blocks(int team) {
     const auto cut = [&](long long n_items, int x) { return static_cast<int>(n_items * x / slices); };
     const long long n_bonded = (d_.nt + kPairBlock - 1) / kPairBlock;
     for (int x = 0; x < slices; ++x) {
-        for (int c = cut(n_bonded, x); c < cut(n_bonded, x + 1); ++c) blocks.push_back(make_int2(-1, c * kPairBlock));
+        for (int c = cut(n_bonded, x); c < cut(n_bonded, x + 1); ++c) blocks.push_back(make_int4(-1, c * kPairBlock, 0, 0));
         for (int g = 0; g < d_.ngroups; ++g) {
             const long long n_items = (group_member_count_[g] + rpb - 1) / rpb;
+            const int stride = host_groups_[g].stride;
             for (int c = cut(n_items, x); c < cut(n_items, x + 1); ++c)
-                blocks.push_back(make_int2(g, group_member_begin_[g] + c * rpb));
+                blocks.push_back(make_int4(g, group_member_begin_[g] + c * rpb,
+                                           static_cast<int>(group_list_base_[g] + static_cast<long long>(c) * rpb * stride),
+                                           stride << 6 | std::min(rpb, group_member_count_[g] - c * rpb)));
         }
     }
     // the block table buffer is reallocated only when it grows
-    static_assert(sizeof(int2) == 8, "int2 layout");
-    if (static_cast<int>(blocks.size()) > d_.n_pair_blocks || !d_.pair_blocks) d_.pair_blocks = dalloc<int2>(blocks.size());
+    static_assert(sizeof(int4) == 16, "int4 layout");
+    if (static_cast<int>(blocks.size()) > d_.n_pair_blocks || !d_.pair_blocks) d_.pair_blocks = dalloc<int4>(blocks.size());
     upload(d_.pair_blocks, blocks);
     d_.n_pair_blocks = static_cast<int>(blocks.size());
     drop_graphs();
@@ -1128,7 +1131,9 @@ void Engine::restore() {
 void Engine::layout_rows() {
     std::vector<int> row_start(std::max(d_.nm, 1), 0);
     long long total = 0;
+    group_list_base_.clear();
     for (const DevPairGroup& G : host_groups_) {
+        group_list_base_.push_back(total);
         for (int r = 0; r < G.member_count; ++r) {
             if (total > std::numeric_limits<int>::max() - G.stride)
                 throw Error(OCM_ERR_OOM, "neighbor list exceeds 2^31 entries");
@@ -1177,7 +1182,7 @@ void Engine::grow_rows() {
     upload(d_.groups, host_groups_);
     check_hip(hipMemset(d_.group_need, 0, sizeof(int) * std::max(ng, 1)), "memset");
     layout_rows();
-    drop_graphs();
+    build_pair_blocks(d_.team);   // the entries carry the rows' list slots
 }
 
 // Device error words are cleared after every read.  Flags raised by a force

@@ -168,6 +168,7 @@ private:
     std::vector<int> group_member_begin_, group_member_count_;
     std::vector<DevPairGroup> host_groups_;
     std::vector<long long> group_list_estimate_;
+    std::vector<long long> group_list_base_;   // first list slot of each group's rows
     std::vector<uint32_t> sys_group_mask_;
     std::vector<int> sys_status_;
     std::vector<int> err_carry_;     // flags of evaluations outside a chunk, reported with the next one

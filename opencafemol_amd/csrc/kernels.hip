@@ -65,6 +65,28 @@ __device__ inline T warp_sum(T v, int width) {
     return v;
 }
 
+// Sum of a 64-bit word over teams of 4 to 64 lanes (aligned within the
+// wavefront), in every lane.  Within 16 lanes by data-parallel-primitive moves
+// (swap in pairs, swap pairs, mirror 8, mirror 16), a few cycles each, where a
+// shuffle is an LDS round trip of ~100; whole numbers, so any order.
+template <int CTRL>
+__device__ __forceinline__ long long dpp_add(long long v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(v >> 32), CTRL, 0xF, 0xF, true);
+    return v + ((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+template <int TEAM>
+__device__ __forceinline__ long long team_sum(long long v) {
+    static_assert(TEAM >= 4 && TEAM <= 64, "teams of 4 to 64 lanes");
+    v = dpp_add<0xB1>(v);                       // quad_perm [1, 0, 3, 2]
+    v = dpp_add<0x4E>(v);                       // quad_perm [2, 3, 0, 1]
+    if (TEAM >= 8) v = dpp_add<0x141>(v);       // row_half_mirror
+    if (TEAM >= 16) v = dpp_add<0x140>(v);      // row_mirror
+    if (TEAM >= 32) v += __shfl_xor(v, 16, 64);
+    if (TEAM >= 64) v += __shfl_xor(v, 32, 64);
+    return v;
+}
+
 // XCD-sliced walk of the pair kernel's block table (batches of many
 // systems).  Workgroups are dispatched to the device's 8 XCDs round-robin,
 // and each XCD has its own L2; workgroup b takes entries of slice b % 8, one
@@ -1754,8 +1776,8 @@ __device__ __forceinline__ int pair_spec(int kinds, bool periodic, const PairK<f
 // gathers in flight; the autotuner picks).
 template <int TEAM, int SPEC, int U>
 __device__ __forceinline__ void force_row(const RowGeom& g, int kinds, const PairK<float>& Kf, const RowType& rt,
-                                          const PairRec& ri, int beg, int cnt, int lane,
-                                          const PairRec* __restrict__ rec, int nrec, const int* __restrict__ col,
+                                          const PairRec& ri, const int* __restrict__ crow, int cnt, int lane,
+                                          const PairRec* __restrict__ rec, int nrec, int (&cn)[U],
                                           const float* __restrict__ lds_types, RowAcc& acc) {
     // A round covers 4*TEAM entries of the row; lane l takes entries l, l+T,
     // l+2T, l+3T of it, so the lanes of one gather read neighbouring entries,
@@ -1767,11 +1789,8 @@ __device__ __forceinline__ void force_row(const RowGeom& g, int kinds, const Pai
     // round computes.
     // (the next round's loads stay conditional here: clamped unconditional
     // loads, as in the prune, measured 4-6% slower in this loop)
-    const int* crow = col + beg;
+    // crow: the row's entries; cn: the first round's, loaded by the caller.
     const __amdgpu_buffer_rsrc_t rs = rec_rsrc(rec, nrec);
-    int cn[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) cn[u] = lane + u * TEAM < cnt ? crow[lane + u * TEAM] : -1;
     for (int base = 0; base < cnt; base += U * TEAM) {
         int cs[U];
 #pragma unroll
@@ -1813,11 +1832,9 @@ __device__ __forceinline__ void force_row(const RowGeom& g, int kinds, const Pai
 template <int TEAM, bool F32>
 __device__ __forceinline__ void prune_row(const DevPairGroup& G, int row, int lane, unsigned long long team_lanes,
                                           const PairRec* __restrict__ rec,
-                                          const float4* __restrict__ rec32, const int* __restrict__ row_start,
-                                          const int* __restrict__ row_count, const int* __restrict__ col,
-                                          int* __restrict__ row_count_w, int* __restrict__ col_w, int nrec) {
-    const int beg = row_start[row];
-    const int cnt = row_count[row];
+                                          const float4* __restrict__ rec32, int cnt, const int* __restrict__ crow,
+                                          int (&cs)[4], int (&cn)[4], int* __restrict__ row_count_w,
+                                          int* __restrict__ wrow, int nrec) {
     double xi = 0, yi = 0, zi = 0;
     float4 qi = make_float4(0.f, 0.f, 0.f, 0.f);
     if (F32) qi = rec32[row];
@@ -1834,8 +1851,6 @@ __device__ __forceinline__ void prune_row(const DevPairGroup& G, int row, int la
         if (lane == 0) row_count_w[row] = 0;
         return;
     }
-    const int* crow = col + beg;
-    int* wrow = col_w + beg;
     const __amdgpu_buffer_rsrc_t rs32 = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<float4*>(rec32), 0, F32 ? nrec * 16 : 0, 0x00020000);
     const __amdgpu_buffer_rsrc_t rs = rec_rsrc(rec, F32 ? 0 : nrec);
@@ -1843,12 +1858,7 @@ __device__ __forceinline__ void prune_row(const DevPairGroup& G, int row, int la
         // software-pipelined: round r's tests run while round r+1's gathers
         // and round r+2's column indices are in flight (the kernel has few
         // wavefronts per SIMD to hide a gather behind)
-        int cs[4], cn[4];
         float4 qj[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) cs[u] = next_col(crow, lane + u * TEAM, cnt);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) cn[u] = next_col(crow, 4 * TEAM + lane + u * TEAM, cnt);
 #pragma unroll
         for (int u = 0; u < 4; ++u) qj[u] = load_rec32(rs32, cs[u]);
         for (int base = 0; base < cnt; base += 4 * TEAM) {
@@ -1878,40 +1888,24 @@ __device__ __forceinline__ void prune_row(const DevPairGroup& G, int row, int la
             for (int u = 0; u < 4; ++u) { cs[u] = cn[u]; cn[u] = cn2[u]; qj[u] = qn[u]; }
         }
     }
-    int cn[4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) cn[u] = next_col(crow, lane + u * TEAM, cnt);
     for (int base = 0; base < (F32 ? 0 : cnt); base += 4 * TEAM) {
-        const int cs[4] = {cn[0], cn[1], cn[2], cn[3]};
         double px[4], py[4], pz[4];
-        float4 qj[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             // padding (-1) reads past the buffer's range: zeros, and keep is false
-            if (F32) qj[u] = load_rec32(rs32, cs[u]);
-            else {
-                const PairRec r = load_rec(rs, cs[u]);
-                px[u] = r.x; py[u] = r.y; pz[u] = r.z;
-            }
+            const PairRec r = load_rec(rs, cs[u]);
+            px[u] = r.x; py[u] = r.y; pz[u] = r.z;
         }
+        int cn2[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) cn[u] = next_col(crow, base + 4 * TEAM + lane + u * TEAM, cnt);
+        for (int u = 0; u < 4; ++u) cn2[u] = next_col(crow, base + 8 * TEAM + lane + u * TEAM, cnt);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            bool in;
-            if (F32) {
-                float dx = qj[u].x - qi.x, dy = qj[u].y - qi.y, dz = qj[u].z - qi.z;
-                dx = fmaf(-fbx, rintf(dx * fibx), dx);
-                dy = fmaf(-fby, rintf(dy * fiby), dy);
-                dz = fmaf(-fbz, rintf(dz * fibz), dz);
-                in = fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < rin2f;
-            } else {
-                const double dx = min_image(px[u] - xi, G.box[0], G.inv_box[0]);
-                const double dy = min_image(py[u] - yi, G.box[1], G.inv_box[1]);
-                const double dz = min_image(pz[u] - zi, G.box[2], G.inv_box[2]);
-                in = dist2(dx, dy, dz) < G.rin2;
-            }
+            const double dx = min_image(px[u] - xi, G.box[0], G.inv_box[0]);
+            const double dy = min_image(py[u] - yi, G.box[1], G.inv_box[1]);
+            const double dz = min_image(pz[u] - zi, G.box[2], G.inv_box[2]);
+            const bool in = dist2(dx, dy, dz) < G.rin2;
             // entry base + u*T + l precedes base + u*T + l' for l < l'; the
             // wave mask is the AND of the two tests' own masks
             const bool valid = cs[u] >= 0, keep = valid & in;
@@ -1922,6 +1916,8 @@ __device__ __forceinline__ void prune_row(const DevPairGroup& G, int row, int la
             if (keep) wrow[n + pos] = cs[u];
             n += __popcll(m);
         }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { cs[u] = cn[u]; cn[u] = cn2[u]; }
     }
     if (lane == 0) {
         int p = n;
@@ -1948,20 +1944,32 @@ __global__ __launch_bounds__(kPairBlock) void k_prune(int nm, const DevPairGroup
     const int lane = threadIdx.x % TEAM;
     const int row = static_cast<int>((static_cast<long long>(blockIdx.x) * kPairBlock + threadIdx.x) / TEAM);
     if (row >= nm) return;   // whole teams leave together
-    const DevPairGroup& G = groups[member_group[row]];
-    if (G.periodic) prune_row<TEAM, true>(G, row, lane, team_lanes, rec, rec32, row_start, row_count, col,
-                                          row_count_w, col_w, nm);
-    else prune_row<TEAM, false>(G, row, lane, team_lanes, rec, rec32, row_start, row_count, col,
-                                row_count_w, col_w, nm);
+    // the row's extent first, then its first two rounds of entries beside the
+    // group's constants (as in k_pair: the fewest round trips in turn)
+    const int gid = member_group[row];
+    const int beg = row_start[row], cnt = row_count[row];
+    const int* crow = col + beg;
+    int cs[4], cn[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int e = lane + u * TEAM;
+        const int a = crow[max(min(e, cnt - 1), 0)], b = crow[max(min(e + 4 * TEAM, cnt - 1), 0)];
+        cs[u] = e < cnt ? a : -1;
+        cn[u] = e + 4 * TEAM < cnt ? b : -1;
+    }
+    const DevPairGroup& G = groups[gid];
+    if (G.periodic) prune_row<TEAM, true>(G, row, lane, team_lanes, rec, rec32, cnt, crow, cs, cn, row_count_w,
+                                          col_w + beg, nm);
+    else prune_row<TEAM, false>(G, row, lane, team_lanes, rec, rec32, cnt, crow, cs, cn, row_count_w, col_w + beg,
+                                nm);
 }
 
 // At least 5 waves per SIMD (<= 96 VGPRs): the record gathers need the latency hiding.
 // SLICED: walk the table in XCD slices (xcd_walk); otherwise a plain stride.
 template <int TEAM, bool SLICED, int U>
 __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5))) void k_pair(
-    const DevPairGroup* __restrict__ groups, const int2* __restrict__ blocks,
-    const PairRec* __restrict__ rec, const int* __restrict__ row_start,
-    const int* __restrict__ row_count, const int* __restrict__ col,
+    const DevPairGroup* __restrict__ groups, const int4* __restrict__ blocks,
+    const PairRec* __restrict__ rec, const int* __restrict__ row_count, const int* __restrict__ col,
     const float* __restrict__ types_f, ForceBuf out,
     uint32_t gmask, int* __restrict__ err, int nblocks, int nrec,
     unsigned long long* __restrict__ stamp, BondedArgs bd) {
@@ -1975,7 +1983,8 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
     const XcdWalk walk = SLICED ? xcd_walk(nblocks) : XcdWalk{static_cast<int>(blockIdx.x), nblocks,
                                                               static_cast<int>(gridDim.x)};
     for (int bi = walk.first; bi < walk.end; bi += walk.stride) {
-    const int2 bt = blocks[bi];
+    // {group, first row, where its list starts, list slots per row << 6 | rows}
+    const int4 bt = blocks[bi];
     if (bt.x < 0) {
         // a chunk of bonded terms, one per thread: their gathers and atomics
         // overlap the pair rows of the other workgroups
@@ -1992,6 +2001,24 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
         }
         continue;
     }
+    // The table entry says all that the row's own loads need, so they go out
+    // at once -- its record, its length and its first entries, read within
+    // the row's slots and masked when the length is there -- beside the
+    // group's constants and type rows, which nothing waits for in turn.  On
+    // systems of a few thousand beads a launch is this chain of memory round
+    // trips and little else: with the entry, the group, the type rows, the
+    // row's extent and its entries waited for one after another, a step of a
+    // 2,100-bead slab took 12.9 us, now 11.8 (14,000 beads: 21.9 and 21.1).
+    const int lane = threadIdx.x % TEAM;
+    const int r = threadIdx.x / TEAM, stride = bt.w >> 6;
+    const bool has_row = r < (bt.w & 63);
+    const int row = bt.y + (has_row ? r : 0);
+    const PairRec ri = rec[row];
+    const int cnt_row = row_count[row];
+    const int* crow = col + bt.z + static_cast<size_t>(row - bt.y) * stride;
+    int cn[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) cn[u] = crow[min(lane + u * TEAM, stride - 1)];
     const DevPairGroup& G = groups[bt.x];
     const RowGeom geo{G.box[0], G.box[1], G.box[2], G.inv_box[0], G.inv_box[1], G.inv_box[2], G.rc2, G.rin2,
                       G.periodic != 0};
@@ -2004,42 +2031,34 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
         loaded = bt.x;
     }
     const int kinds = group_kinds(G, gmask);
-    const int lane = threadIdx.x % TEAM;
-    const int row = bt.y + threadIdx.x / TEAM;
-    const int row_end = G.member_begin + G.member_count;
     RowAcc acc;
     int bead_i = -1;
-    if (row < row_end && kinds) {
-        const PairRec ri = rec[row];
+    if (has_row && kinds) {
         bead_i = ri.bead;
-        const int beg = row_start[row], cnt = row_count[row];
+        const int cnt = cnt_row;
+#pragma unroll
+        for (int u = 0; u < U; ++u) cn[u] = lane + u * TEAM < cnt ? cn[u] : -1;
         const int ti = ri.type & 0xFFFF;
         const RowType rt = row_type(lds_types + ti * kTypeStride);
         // the group's kind selects the loop (uniform over the workgroup)
         switch (pair_spec(kinds, geo.periodic, Kf)) {
         case kSpecExvPeriodic:
-            force_row<TEAM, kSpecExvPeriodic, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                                 lds_types, acc);
+            force_row<TEAM, kSpecExvPeriodic, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
             break;
         case kSpecExvOpen:
-            force_row<TEAM, kSpecExvOpen, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                             lds_types, acc);
+            force_row<TEAM, kSpecExvOpen, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
             break;
         case kSpecDh:
-            force_row<TEAM, kSpecDh, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                        lds_types, acc);
+            force_row<TEAM, kSpecDh, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
             break;
         case kSpecLjShared:
-            force_row<TEAM, kSpecLjShared, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                              lds_types, acc);
+            force_row<TEAM, kSpecLjShared, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
             break;
         case kSpecSolo:
-            force_row<TEAM, kSpecSolo, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                          lds_types, acc);
+            force_row<TEAM, kSpecSolo, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
             break;
         default:
-            force_row<TEAM, kSpecGeneric, U>(geo, kinds, Kf, rt, ri, beg, cnt, lane, rec, nrec, col,
-                                             lds_types, acc);
+            force_row<TEAM, kSpecGeneric, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
             break;
         }
     }
@@ -2047,9 +2066,9 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
     long long ax = static_cast<long long>(acc.ux - off);
     long long ay = static_cast<long long>(acc.uy - off);
     long long az = static_cast<long long>(acc.uz - off);
-    ax = warp_sum(ax, TEAM);
-    ay = warp_sum(ay, TEAM);
-    az = warp_sum(az, TEAM);
+    ax = team_sum<TEAM>(ax);
+    ay = team_sum<TEAM>(ay);
+    az = team_sum<TEAM>(az);
     if (lane == 0 && bead_i >= 0) {
         atomicAdd(reinterpret_cast<unsigned long long*>(&out.fx[bead_i]), static_cast<unsigned long long>(ax));
         atomicAdd(reinterpret_cast<unsigned long long*>(&out.fy[bead_i]), static_cast<unsigned long long>(ay));
@@ -2074,7 +2093,7 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
 // frame takes 519 us.
 template <int TEAM>
 __global__ __launch_bounds__(kPairBlock) void k_pair_energy(
-    const DevPairGroup* __restrict__ groups, const int2* __restrict__ blocks, const PairRec* __restrict__ rec,
+    const DevPairGroup* __restrict__ groups, const int4* __restrict__ blocks, const PairRec* __restrict__ rec,
     const int* __restrict__ row_start, const int* __restrict__ row_count, const int* __restrict__ col,
     const double* __restrict__ types_d, long long* __restrict__ energy, int ecopies, int estride, uint32_t gmask,
     int* __restrict__ err, int nblocks) {
@@ -2098,7 +2117,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pair_energy(
         ae0 = ae1 = ae2 = ae3 = 0;
     };
     for (int bi = static_cast<int>(blockIdx.x); bi < nblocks; bi += static_cast<int>(gridDim.x)) {
-        const int2 bt = blocks[bi];
+        const int4 bt = blocks[bi];
         if (bt.x < 0) continue;   // bonded terms: k_bonded
         const DevPairGroup& G = groups[bt.x];
         const int kinds = group_kinds(G, gmask);
@@ -2923,11 +2942,11 @@ static void pair_dispatch(const DevPtrs& d, hipStream_t st, const ForceBuf& f, u
     const dim3 grid(std::min(d.n_pair_blocks, d.pair_grid)), block(kPairBlock);
 #define OCM_PAIR(T, U)                                                                                       \
     if (d.xcd_sliced)                                                                                        \
-        k_pair<T, true, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, count, col, \
+        k_pair<T, true, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, count, col, \
                                                      d.types_f, f, groups, d.err, d.n_pair_blocks, d.nm,     \
                                                      stamp, bd);                                             \
     else                                                                                                     \
-        k_pair<T, false, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, d.row_start, count, col, \
+        k_pair<T, false, U><<<grid, block, lds, st>>>(d.groups, d.pair_blocks, d.rec, count, col, \
                                                       d.types_f, f, groups, d.err, d.n_pair_blocks, d.nm,    \
                                                       stamp, bd)
     if (d.pair_u == 2) {

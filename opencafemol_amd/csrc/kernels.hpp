@@ -68,7 +68,9 @@ struct DevPtrs {
     float* types_f = nullptr;
     double* types_d = nullptr;
     int max_types = 0;
-    int2* pair_blocks = nullptr;   // (group, first slot) per pair-kernel block
+    // per pair-kernel block {group, first row, its list start, list slots per row << 6 | rows},
+    // or {-1, first bonded term}
+    int4* pair_blocks = nullptr;
     int n_pair_blocks = 0;
     int xcd_sliced = 0;            // pair_blocks holds 8 contiguous XCD slices of equal work mix (batches of many systems)
     int team = 16;
