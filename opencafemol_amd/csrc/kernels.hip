@@ -1498,12 +1498,19 @@ __device__ inline RowType row_type(const float* __restrict__ t) {
 // switch polynomial is evaluated at x = max(0, (r - rsw)/w), where x = 0 gives
 // S = 1 and dS = 0, the unswitched value exactly.
 // (1/r is left in *ir_out when the kinds need it, else 0.)
+// Open Ashbaugh-Hatch groups take s^12 - s^6 and r - rsw from rounded s^12 and
+// r; the periodic loop's fused forms round once less.  Each kind of boundary
+// keeps the rounding its trajectories have always had (open_lj).
+__device__ __forceinline__ float sub_rounded(float a, float b) {
+#pragma clang fp contract(off)
+    return a - b;
+}
 __device__ __forceinline__ bool pair_force_has_ir(int kinds, bool lsw) {
     return (kinds & (kDh | kIsolf)) || ((kinds & (kLja | kUlja)) && lsw);
 }
 __device__ __forceinline__ float pair_force(int kinds, bool shared, bool lsw, const PairK<float>& G,
                                             const RowType& ti, const float* __restrict__ tj, float r2,
-                                            float* ir_out = nullptr) {
+                                            float* ir_out = nullptr, bool open_lj = false) {
     const float ir2 = __builtin_amdgcn_rcpf(r2);
     float f = 0.f, r = 0.f, ir = 0.f;
     if (pair_force_has_ir(kinds, lsw)) {
@@ -1534,11 +1541,11 @@ __device__ __forceinline__ float pair_force(int kinds, bool shared, bool lsw, co
         const float er = ti.er + lj.x, ea = ti.ea + lj.z;
         const bool inner = th2 - r2 >= 0.f, outer = r2 - th2 >= 0.f;
         f += inner ? er * X : 0.f;
-        float u = outer ? 4.f * ea * (s12 - s6) : 0.f;
+        float u = outer ? 4.f * ea * (open_lj ? sub_rounded(s12, s6) : s12 - s6) : 0.f;
         float du = outer ? ea * X : 0.f;
         u = inner ? u - ea : u;
         if (lsw) {
-            const float x = fmaxf((r - G.lja_rsw) * G.lja_inv_sw, 0.f);
+            const float x = fmaxf((open_lj ? sub_rounded(r, G.lja_rsw) : r - G.lja_rsw) * G.lja_inv_sw, 0.f);
             const float x2 = x * x, x3 = x2 * x;
             const float S = 1.f - x3 * (10.f - 15.f * x + 6.f * x2);
             const float dS = -30.f * x2 * (1.f - x) * (1.f - x) * G.lja_inv_sw;
@@ -1654,8 +1661,12 @@ struct BondedArgs {
 // has no branches and the four entries of a round interleave.
 // kSpecGeneric covers any mix of the four round kinds (EXV, DH, LJ
 // repulsive, LJ attractive), kSpecSolo the kinds that sit alone in a group.
+// The open variants skip the minimum image.
 constexpr int kSpecGeneric = 0, kSpecExvPeriodic = 1, kSpecExvOpen = 2, kSpecDh = 3, kSpecLjShared = 4,
-              kSpecSolo = 5;
+              kSpecSolo = 5, kSpecDhOpen = 6, kSpecLjSharedOpen = 7;
+constexpr bool spec_dh(int spec) { return spec == kSpecDh || spec == kSpecDhOpen; }
+constexpr bool spec_lj(int spec) { return spec == kSpecLjShared || spec == kSpecLjSharedOpen; }
+constexpr bool spec_open(int spec) { return spec == kSpecExvOpen || spec == kSpecDhOpen || spec == kSpecLjSharedOpen; }
 
 // Raw buffer over the pair records: 32-bit offsets instead of 64-bit
 // addresses, and a read past the end (the -1 padding entries) returns zeros
@@ -1715,7 +1726,7 @@ __device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const 
                                              double& dz, int& bad) {
     // a group without a box has inverse box 0, for which the minimum
     // image is the identity
-    if (SPEC == kSpecGeneric || SPEC == kSpecSolo ? g.periodic : SPEC != kSpecExvOpen) {
+    if (SPEC == kSpecGeneric || SPEC == kSpecSolo ? g.periodic : !spec_open(SPEC)) {
         dx = min_image(dx, g.bx, g.ibx);
         dy = min_image(dy, g.by, g.iby);
         dz = min_image(dz, g.bz, g.ibz);
@@ -1725,8 +1736,8 @@ __device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const 
     const float r2f = in ? static_cast<float>(r2) : 1.0f;
     float f, ir = 0.f;
     if (SPEC == kSpecExvPeriodic || SPEC == kSpecExvOpen) f = pair_force(kExv, false, false, Kf, rt, tfj, r2f);
-    else if (SPEC == kSpecDh) f = pair_force(kDh, false, false, Kf, rt, tfj, r2f, &ir);
-    else if (SPEC == kSpecLjShared) f = pair_force(kLjr | kLja, true, true, Kf, rt, tfj, r2f, &ir);
+    else if (spec_dh(SPEC)) f = pair_force(kDh, false, false, Kf, rt, tfj, r2f, &ir);
+    else if (spec_lj(SPEC)) f = pair_force(kLjr | kLja, true, true, Kf, rt, tfj, r2f, &ir, SPEC == kSpecLjSharedOpen);
     else if (SPEC == kSpecSolo) f = pair_force(kinds & ~(kExv | kDh | kLjr | kLja), false, Kf.lja_switch, Kf, rt,
                                                tfj, r2f);
     else f = pair_force(kinds & (kExv | kDh | kLjr | kLja), Kf.lj_shared, Kf.lja_switch, Kf, rt, tfj, r2f);
@@ -1738,7 +1749,7 @@ __device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const 
     const bool ok = f * f * r2f < kPairLimit * kPairLimit;
     bad |= in && !ok;
     float gg;
-    if (SPEC == kSpecDh || SPEC == kSpecLjShared) {
+    if (spec_dh(SPEC) || spec_lj(SPEC)) {
         const float cl = copysignf(0.999f * kPairLimit, f) * ir;
         gg = ok ? f : (f == f ? cl : 0.0f);
     } else {
@@ -1764,8 +1775,8 @@ __device__ __forceinline__ int group_kinds(const DevPairGroup& G, uint32_t gmask
 // The pair kernel's spec (specialized row loop) of a group with these kinds.
 __device__ __forceinline__ int pair_spec(int kinds, bool periodic, const PairK<float>& Kf) {
     if (kinds == kExv) return periodic ? kSpecExvPeriodic : kSpecExvOpen;
-    if (kinds == kDh && periodic) return kSpecDh;
-    if (kinds == (kLjr | kLja) && Kf.lj_shared && Kf.lja_switch && periodic) return kSpecLjShared;
+    if (kinds == kDh) return periodic ? kSpecDh : kSpecDhOpen;
+    if (kinds == (kLjr | kLja) && Kf.lj_shared && Kf.lja_switch) return periodic ? kSpecLjShared : kSpecLjSharedOpen;
     if (kinds & ~(kExv | kDh | kLjr | kLja)) return kSpecSolo;
     return kSpecGeneric;
 }
@@ -2053,6 +2064,13 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
             break;
         case kSpecLjShared:
             force_row<TEAM, kSpecLjShared, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
+            break;
+        case kSpecDhOpen:
+            force_row<TEAM, kSpecDhOpen, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
+            break;
+        case kSpecLjSharedOpen:
+            force_row<TEAM, kSpecLjSharedOpen, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types,
+                                                  acc);
             break;
         case kSpecSolo:
             force_row<TEAM, kSpecSolo, U>(geo, kinds, Kf, rt, ri, crow, cnt, lane, rec, nrec, cn, lds_types, acc);
@@ -2549,6 +2567,8 @@ __device__ __forceinline__ void res_forces(const ResArgs& a, const ResSys& R, co
         case kSpecExvOpen: res_pairs<kSpecExvOpen, T>(a, K, off, L, bad); break;
         case kSpecDh: res_pairs<kSpecDh, T>(a, K, off, L, bad); break;
         case kSpecLjShared: res_pairs<kSpecLjShared, T>(a, K, off, L, bad); break;
+        case kSpecDhOpen: res_pairs<kSpecDhOpen, T>(a, K, off, L, bad); break;
+        case kSpecLjSharedOpen: res_pairs<kSpecLjSharedOpen, T>(a, K, off, L, bad); break;
         case kSpecSolo: res_pairs<kSpecSolo, T>(a, K, off, L, bad); break;
         default: res_pairs<kSpecGeneric, T>(a, K, off, L, bad); break;
         }
