@@ -103,7 +103,7 @@ struct DevPairGroup {
 };
 
 // Resident stepping (small systems, one workgroup per system, whole chunks
-// on chip): per system, its bonded terms (bead indices local to the system)
+// on chip): per system, its bonded terms (bead indices local to the system, times 3)
 // and its pair groups, whose FP32 type rows are staged together in LDS.
 constexpr int kResMaxBeads = 1024;      // beads per system (local indices fit 10 bits)
 constexpr int kResMaxGroups = 8;        // pair groups per system
@@ -112,7 +112,9 @@ constexpr int kResMaxTypeRows = 64;     // staged type rows per system (6 bits)
 // wrapped into boxes of at most kResWide nm, open systems' relative to bead 0
 // (a build that finds one beyond kResWide tests that build's pairs in FP64).
 constexpr double kResWide = 1000.0;
-constexpr int kResMaxSeg = 9;   // bonded kinds 1-9: one segment each
+// A unit is up to 64 bonded terms of one kind: bits 0-19 the first term, 20-25
+// the terms less one, 26-31 its cost in kResUnitCost.
+constexpr int kResUnitCost = 16;
 struct ResSys {
     int sys;          // DevSys index
     int nb;           // beads
@@ -121,10 +123,8 @@ struct ResSys {
     int g0, ng;       // resident pair groups [g0, g0 + ng)
     int row0, nrow;   // staged type rows [row0, row0 + nrow) of the resident row array
     int ex0, exn;     // the groups' exclusion tables: words [ex0, ex0 + exn) of the resident exclusion array
-    // the terms in runs of one kind: run q is terms [seg_t[q], seg_t[q] + seg_n[q])
-    // of the system's own (kind-ordered) list
-    int nseg;
-    int seg_t[kResMaxSeg], seg_n[kResMaxSeg];
+    int u0, nu;       // units of its bonded terms: words [u0, u0 + nu) of the resident unit table
+    int ucost;        // their summed cost
 };
 // A group's exclusions in member order (members follow bead order), for the
 // in-kernel build, which tests member pairs (i, j > i): per member a mask

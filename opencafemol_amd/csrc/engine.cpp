@@ -796,6 +796,7 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     std::vector<BTerm> rterms;
     std::vector<float> rows;
     std::vector<int> rexcl;
+    std::vector<uint32_t> units;
     // per bead: the smallest (skin/2)^2 of its groups' resident lists
     std::vector<double> res_hs2(static_cast<size_t>(d_.nb), std::numeric_limits<double>::max());
     std::vector<std::vector<int>> sys_terms(nsys);
@@ -813,20 +814,32 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
         R.b0 = bead_begin_[s];
         R.t0 = static_cast<int>(rterms.size());
         R.nt = static_cast<int>(sys_terms[s].size());
-        R.nseg = 0;
         for (int t : sys_terms[s]) {   // kind order is kept within the system
             BTerm T = terms[t];
             for (int k = 0; k < 4; ++k)
-                if (T.idx[k] >= 0) T.idx[k] -= R.b0;
-            const int local = static_cast<int>(rterms.size()) - R.t0;
-            if (R.nseg == 0 || rterms.back().kind != T.kind) {
-                if (R.nseg == kResMaxSeg) throw Error(OCM_ERR_INVALID, "resident terms are not in kind order");
-                R.seg_t[R.nseg] = local;
-                R.seg_n[R.nseg] = 0;
-                ++R.nseg;
-            }
-            ++R.seg_n[R.nseg - 1];
+                if (T.idx[k] >= 0) T.idx[k] = 3 * (T.idx[k] - R.b0);
             rterms.push_back(T);
+        }
+        if (R.nt >= 1 << 20) return;   // a unit word's first term has 20 bits
+        // units of up to 64 terms of one kind, costly kinds first: estimated
+        // VALU instructions of a term by kind
+        static const int cost[10] = {0, 90, 100, 90, 190, 290, 250, 310, 110, 300};
+        std::vector<std::pair<int, uint32_t>> unit;
+        for (int t = 0; t < R.nt;) {
+            const int kind = rterms[R.t0 + t].kind;
+            int n = 1;
+            while (n < 64 && t + n < R.nt && rterms[R.t0 + t + n].kind == kind) ++n;
+            unit.emplace_back(-cost[kind], static_cast<uint32_t>(t) | static_cast<uint32_t>(n - 1) << 20 |
+                                               static_cast<uint32_t>(cost[kind] / kResUnitCost) << 26);
+            t += n;
+        }
+        std::stable_sort(unit.begin(), unit.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
+        R.u0 = static_cast<int>(units.size());
+        R.nu = static_cast<int>(unit.size());
+        R.ucost = 0;
+        for (const auto& q : unit) {
+            units.push_back(q.second);
+            R.ucost += static_cast<int>(q.second >> 26);
         }
         R.g0 = static_cast<int>(grp.size());
         R.ng = static_cast<int>(sys_groups[s].size());
@@ -887,7 +900,7 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     }
     // a step's work (terms, list entries, noise) is dealt over all threads:
     // 1024 of them keep every thread's share short
-    d_.res_threads = 1024;
+    d_.res_threads = kResThreads;
     d_.res_nbs = (max_n + 63) & ~63;
     // LDS: what one system's step reads, as far as it fits.  Up to one
     // workgroup per CU the whole 160 KB may go to one; beyond that half, so
@@ -912,15 +925,17 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     // exclusion tables are staged whole; they are small (chains exclude near
     // neighbours, which are mask bits)
     d_.res_ex_cap = max_ex;
-    const size_t fixed = resident_lds_bytes(d_.res_nbs, 0, 0, d_.res_ex_cap);
+    d_.res_unit_cap = 0;
+    for (const ResSys& R : tab) d_.res_unit_cap = std::max(d_.res_unit_cap, R.nu);
+    const size_t fixed = resident_lds_bytes(d_.res_nbs, 0, 0, d_.res_ex_cap, d_.res_unit_cap);
     if (fixed > budget) { d_.res_n = 0; return; }
     const size_t room = budget - fixed;
     d_.res_list_cap = static_cast<int>(std::min<long long>({max_pairs, kResListLdsMax,
                                                             static_cast<long long>(room / sizeof(uint32_t))}));
     d_.res_term_cap = static_cast<int>(std::min<size_t>(static_cast<size_t>(max_nt),
                                                         (room - d_.res_list_cap * sizeof(uint32_t)) / sizeof(BTerm)));
-    const size_t lds = resident_lds_bytes(d_.res_nbs, d_.res_term_cap, d_.res_list_cap, d_.res_ex_cap);
-    check_hip(resident_prepare(d_.res_threads, lds), "hipFuncSetAttribute (resident LDS)");
+    const size_t lds = resident_lds_bytes(d_.res_nbs, d_.res_term_cap, d_.res_list_cap, d_.res_ex_cap, d_.res_unit_cap);
+    check_hip(resident_prepare(lds), "hipFuncSetAttribute (resident LDS)");
     d_.res_tab = dalloc<ResSys>(tab.size()); upload(d_.res_tab, tab);
     d_.res_grp = dalloc<ResGroup>(std::max<size_t>(grp.size(), 1));
     if (!grp.empty()) upload(d_.res_grp, grp);
@@ -933,6 +948,8 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     upload(d_.res_hs2, res_hs2);
     d_.res_excl = dalloc<int>(std::max<size_t>(rexcl.size(), 1));
     if (!rexcl.empty()) upload(d_.res_excl, rexcl);
+    d_.res_units = dalloc<uint32_t>(std::max<size_t>(units.size(), 1));
+    if (!units.empty()) upload(d_.res_units, units);
     d_.res_n = nsys;
 }
 

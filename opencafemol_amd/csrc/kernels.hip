@@ -31,18 +31,16 @@ namespace ocm {
 // the float-to-integer conversion is only ever applied to representable values.
 //
 // FP32 values go to fixed point as floor(v * 2^32): floor(v) is the high word
-// and the fraction, scaled by 2^32, the low word.  v - floor(v) is exact except
-// for negative |v| < 1, where it is rounded once (by at most 2^-25); the low
-// word is clamped below 2^32 for the case it rounds up to 1.  Requires |v| < 2^30.
+// (one instruction, V_CVT_FLR_I32_F32) and the fraction, scaled by 2^32, the
+// low word (V_FRACT_F32 keeps it below 1, where v - floor(v) of a tiny
+// negative v would round up to it).  Four instructions a component where the
+// range test, floor, subtraction, clamp and conversions took eleven, the same
+// words for every float below 2^30.  Requires |v| < 2^30.
 __device__ inline long long fix_floor(float v) {
-    const float h = floorf(v);
-    const float l = fminf((v - h) * 4294967296.0f, 4294967040.0f);
-    return (static_cast<long long>(static_cast<int>(h)) << 32) + static_cast<long long>(static_cast<unsigned>(l));
-}
-__device__ inline long long to_fix(float v, int& bad) {
-    const bool ok = fabsf(v) < kFixLimitF;
-    bad |= !ok;
-    return fix_floor(ok ? v : 0.0f);
+    int h;
+    asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(h) : "v"(v));
+    const unsigned l = static_cast<unsigned>(__builtin_amdgcn_fractf(v) * 4294967296.0f);
+    return static_cast<long long>((static_cast<unsigned long long>(static_cast<unsigned>(h)) << 32) | l);
 }
 __device__ inline long long to_fix_d(double v, int& bad) {
     const bool ok = fabs(v) < 1073741824.0;
@@ -333,8 +331,10 @@ __device__ __forceinline__ double half_kick(double v, double h, double f, double
 // step's noise, half a drift.  Fixed (massless) beads keep X and V.  Returns
 // false when a mobile bead's new position is not finite.
 // g holds the step's three N(0,1) samples (gauss3_fast).
-__device__ __forceinline__ bool baoab_bead_g(const DevSys& S, double im, long long F0, long long F1, long long F2,
-                                             const double (&X)[3], const double (&V)[3], int pending,
+// sig: the bead's noise amplitude sqrt(noise_kT / m) (noise_sigma).
+__device__ __forceinline__ double noise_sigma(const DevSys& S, double im) { return sqrt(S.noise_kT * im); }
+__device__ __forceinline__ bool baoab_bead_g(const DevSys& S, double im, double sig, long long F0, long long F1,
+                                             long long F2, const double (&X)[3], const double (&V)[3], int pending,
                                              const double (&g)[3], double (&x)[3], double (&v)[3]) {
     const double f0 = F0 * kFixInv, f1 = F1 * kFixInv, f2 = F2 * kFixInv;
     double v0 = V[0], v1 = V[1], v2 = V[2];
@@ -351,7 +351,6 @@ __device__ __forceinline__ bool baoab_bead_g(const DevSys& S, double im, long lo
     double x0 = fma(S.half_dt, v0, X[0]);
     double x1 = fma(S.half_dt, v1, X[1]);
     double x2 = fma(S.half_dt, v2, X[2]);
-    const double sig = sqrt(S.noise_kT * im);
     v0 = fma(S.c1, v0, sig * g[0]);
     v1 = fma(S.c1, v1, sig * g[1]);
     v2 = fma(S.c1, v2, sig * g[2]);
@@ -372,7 +371,7 @@ __device__ __forceinline__ bool baoab_bead(const DevSys& S, double im, long long
                                            uint32_t lid, double (&x)[3], double (&v)[3]) {
     double g[3];
     gauss3_fast(S.seed, static_cast<uint64_t>(step - S.step_origin), lid, g);
-    return baoab_bead_g(S, im, F0, F1, F2, X, V, pending, g, x, v);
+    return baoab_bead_g(S, im, noise_sigma(S, im), F0, F1, F2, X, V, pending, g, x, v);
 }
 
 // pending != 0: the closing half kick of the previous step is still owed and
@@ -476,7 +475,10 @@ __global__ void k_pack(int nm, const DevPairGroup* __restrict__ groups,
 // skin (widened while the grid would exceed the cells reserved for it).
 // Beads that leave the box before the next build are clamped into the edge
 // cells, which keeps every pair within rl in neighbouring cells.
-constexpr int kOpenGridThreads = 256;
+// One workgroup per group: the reduction is a chain of gathers (member to bead
+// to position), so 1,024 threads take four members at a time with their loads
+// issued together (21,000 members: 53 us with 256 threads one by one, now 13).
+constexpr int kOpenGridThreads = 1024;
 __global__ __launch_bounds__(kOpenGridThreads) void k_open_grid(DevPairGroup* __restrict__ groups,
                                                                 const int* __restrict__ member_bead,
                                                                 const double* __restrict__ px,
@@ -484,29 +486,41 @@ __global__ __launch_bounds__(kOpenGridThreads) void k_open_grid(DevPairGroup* __
                                                                 const double* __restrict__ pz) {
     DevPairGroup& G = groups[blockIdx.x];
     if (!G.open_grid) return;   // uniform over the workgroup
-    __shared__ double red[6][kOpenGridThreads];
+    __shared__ double red[6][kOpenGridThreads / 64];
     double lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
-    for (int m = G.member_begin + threadIdx.x; m < G.member_begin + G.member_count; m += blockDim.x) {
-        const int b = member_bead[m];
-        const double p[3] = {px[b], py[b], pz[b]};
+    const int nmem = G.member_count;
+    for (int m0 = threadIdx.x; m0 < nmem; m0 += 4 * kOpenGridThreads) {
+        int b[4];
+        double p[4][3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
-            if (isfinite(p[d])) { lo[d] = fmin(lo[d], p[d]); hi[d] = fmax(hi[d], p[d]); }
+        for (int u = 0; u < 4; ++u)   // past the end: the last member again
+            b[u] = member_bead[G.member_begin + min(m0 + u * kOpenGridThreads, nmem - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { p[u][0] = px[b[u]]; p[u][1] = py[b[u]]; p[u][2] = pz[b[u]]; }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                if (isfinite(p[u][d])) { lo[d] = fmin(lo[d], p[u][d]); hi[d] = fmax(hi[d], p[u][d]); }
     }
 #pragma unroll
-    for (int d = 0; d < 3; ++d) { red[d][threadIdx.x] = lo[d]; red[3 + d][threadIdx.x] = hi[d]; }
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if (static_cast<int>(threadIdx.x) < w) {
-#pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                red[d][threadIdx.x] = fmin(red[d][threadIdx.x], red[d][threadIdx.x + w]);
-                red[3 + d][threadIdx.x] = fmax(red[3 + d][threadIdx.x], red[3 + d][threadIdx.x + w]);
-            }
+    for (int d = 0; d < 3; ++d)
+        for (int o = 32; o > 0; o >>= 1) {
+            lo[d] = fmin(lo[d], __shfl_xor(lo[d], o, 64));
+            hi[d] = fmax(hi[d], __shfl_xor(hi[d], o, 64));
         }
-        __syncthreads();
+    if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) { red[d][threadIdx.x >> 6] = lo[d]; red[3 + d][threadIdx.x >> 6] = hi[d]; }
     }
+    __syncthreads();
     if (threadIdx.x != 0) return;
+    for (int w = 1; w < kOpenGridThreads / 64; ++w)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            red[d][0] = fmin(red[d][0], red[d][w]);
+            red[3 + d][0] = fmax(red[3 + d][0], red[3 + d][w]);
+        }
     double ext[3], l0[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -1013,21 +1027,45 @@ __global__ void k_scan_add(int* __restrict__ out, int n, const int* __restrict__
 // ----------------------------------------------------------------- bonded
 template <typename R> struct V3T { R x, y, z; };
 
-template <typename R>
-__device__ inline V3T<R> bdisp(const double* __restrict__ px, const double* __restrict__ py,
-                               const double* __restrict__ pz, int i, int j, const DevSys& S, bool pbc) {
-    double dx = px[j] - px[i], dy = py[j] - py[i], dz = pz[j] - pz[i];
-    if (pbc && S.periodic) {
-        dx = min_image(dx, S.box[0], S.inv_box[0]);
-        dy = min_image(dy, S.box[1], S.inv_box[1]);
-        dz = min_image(dz, S.box[2], S.inv_box[2]);
+// Displacements of a term's beads from one to the next (vector k from bead
+// from[k] to bead to[k]).  Every position is read before the first is used and
+// the minimum image has one branch, uniform for systems without a box, so the
+// reads are one wait: a wavefront with one term per lane has nothing else to
+// hide them behind (with a branch and a wait per vector, the dihedral
+// wavefront that bounds a 62-bead chain's step took 3.7 k cycles; with the
+// units dealt from two ends the step went from 2.54 to 1.73 us).
+template <int N>
+__device__ __forceinline__ void bdisps(const double* __restrict__ px, const double* __restrict__ py,
+                                       const double* __restrict__ pz, const int (&from)[N], const int (&to)[N],
+                                       const DevSys& S, bool pbc, V3T<double> (&d)[N]) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+        d[k] = {px[to[k]] - px[from[k]], py[to[k]] - py[from[k]], pz[to[k]] - pz[from[k]]};
+    if (S.periodic) {
+        if (pbc) {
+#pragma unroll
+            for (int k = 0; k < N; ++k)
+                d[k] = {min_image(d[k].x, S.box[0], S.inv_box[0]), min_image(d[k].y, S.box[1], S.inv_box[1]),
+                        min_image(d[k].z, S.box[2], S.inv_box[2])};
+        }
     }
-    return {static_cast<R>(dx), static_cast<R>(dy), static_cast<R>(dz)};
+}
+template <typename R> __device__ inline V3T<R> to_v3(const V3T<double>& d) {
+    return {static_cast<R>(d.x), static_cast<R>(d.y), static_cast<R>(d.z)};
 }
 template <typename R> __device__ inline V3T<R> cross3(V3T<R> a, V3T<R> b) {
     return {a.y * b.z - a.z * b.y, a.z * b.x - a.x * b.z, a.x * b.y - a.y * b.x};
 }
 template <typename R> __device__ inline R dot3(V3T<R> a, V3T<R> b) { return a.x * b.x + a.y * b.y + a.z * b.z; }
+// The force pass's products with their fused operations spelled out, so that
+// a term has the same bits in every kernel it is inlined in.
+template <> __device__ inline V3T<float> cross3(V3T<float> a, V3T<float> b) {
+    return {__builtin_fmaf(a.y, b.z, -(a.z * b.y)), __builtin_fmaf(a.z, b.x, -(a.x * b.z)),
+            __builtin_fmaf(a.x, b.y, -(a.y * b.x))};
+}
+template <> __device__ inline float dot3(V3T<float> a, V3T<float> b) {
+    return __builtin_fmaf(a.z, b.z, __builtin_fmaf(a.x, b.x, a.y * b.y));
+}
 
 template <typename R> __device__ inline R r_sqrt(R v);
 template <> __device__ inline float r_sqrt<float>(float v) { return __builtin_amdgcn_sqrtf(v); }
@@ -1068,8 +1106,18 @@ struct FixV {
 };
 template <typename R>
 __device__ inline FixV fix_v(R gx, R gy, R gz, int& bad) {
-    if constexpr (sizeof(R) == 4) return {to_fix(gx, bad), to_fix(gy, bad), to_fix(gz, bad)};
-    else return {to_fix_d(gx, bad), to_fix_d(gy, bad), to_fix_d(gz, bad)};
+    if constexpr (sizeof(R) == 4) {
+        // one range test for the three (a sum that reaches 2^30 or is not a
+        // number looks at each)
+        if (!(fabsf(gx) + fabsf(gy) + fabsf(gz) < kFixLimitF)) {
+            const bool okx = fabsf(gx) < kFixLimitF, oky = fabsf(gy) < kFixLimitF, okz = fabsf(gz) < kFixLimitF;
+            bad |= !(okx && oky && okz);
+            gx = okx ? gx : R(0);
+            gy = oky ? gy : R(0);
+            gz = okz ? gz : R(0);
+        }
+        return {fix_floor(gx), fix_floor(gy), fix_floor(gz)};
+    } else return {to_fix_d(gx, bad), to_fix_d(gy, bad), to_fix_d(gz, bad)};
 }
 __device__ inline void add_fix(const ForceOut& o, int b, long long x, long long y, long long z) {
     atomicAdd(reinterpret_cast<unsigned long long*>(&o.fx[b]), static_cast<unsigned long long>(x));
@@ -1090,8 +1138,10 @@ __device__ inline void bonded_term(const BTerm& t, const DevSys& S, const double
     R e = 0;
     switch (t.kind) {
     case 1: case 2: case 3: case 8: {  // harmonic bond, Gaussian bond, Go contact, capped Go contact
-        const V3T<double> dd = bdisp<double>(px, py, pz, t.idx[0], t.idx[1], S, pbc);
-        const V3T<R> d = {static_cast<R>(dd.x), static_cast<R>(dd.y), static_cast<R>(dd.z)};
+        V3T<double> dv[1];
+        bdisps<1>(px, py, pz, {t.idx[0]}, {t.idx[1]}, S, pbc, dv);
+        const V3T<double> dd = dv[0];
+        const V3T<R> d = to_v3<R>(dd);
         const double r2d = fma(dd.z, dd.z, fma(dd.y, dd.y, dd.x * dd.x));
         const R r = r_sqrt<R>(static_cast<R>(r2d));
         // r - r0 of the two stiff kinds.  In FP32, r - r0 from an FP32 r
@@ -1141,8 +1191,9 @@ __device__ inline void bonded_term(const BTerm& t, const DevSys& S, const double
         break;
     }
     case 4: case 5: {  // harmonic angle, flexible local angle
-        const V3T<R> a = bdisp<R>(px, py, pz, t.idx[1], t.idx[0], S, pbc);  // x_i - x_j
-        const V3T<R> c = bdisp<R>(px, py, pz, t.idx[1], t.idx[2], S, pbc);  // x_k - x_j
+        V3T<double> dv[2];
+        bdisps<2>(px, py, pz, {t.idx[1], t.idx[1]}, {t.idx[0], t.idx[2]}, S, pbc, dv);
+        const V3T<R> a = to_v3<R>(dv[0]), c = to_v3<R>(dv[1]);   // x_i - x_j, x_k - x_j
         const V3T<R> p = cross3(a, c);
         const R pn = r_sqrt<R>(dot3(p, p));
         const R th = r_atan2<R>(pn, dot3(a, c));
@@ -1185,9 +1236,9 @@ __device__ inline void bonded_term(const BTerm& t, const DevSys& S, const double
         break;
     }
     case 6: case 7: case 9: {  // Gaussian, flexible local and cosine dihedrals
-        const V3T<R> b1 = bdisp<R>(px, py, pz, t.idx[0], t.idx[1], S, pbc);
-        const V3T<R> b2 = bdisp<R>(px, py, pz, t.idx[1], t.idx[2], S, pbc);
-        const V3T<R> b3 = bdisp<R>(px, py, pz, t.idx[2], t.idx[3], S, pbc);
+        V3T<double> dv[3];
+        bdisps<3>(px, py, pz, {t.idx[0], t.idx[1], t.idx[2]}, {t.idx[1], t.idx[2], t.idx[3]}, S, pbc, dv);
+        const V3T<R> b1 = to_v3<R>(dv[0]), b2 = to_v3<R>(dv[1]), b3 = to_v3<R>(dv[2]);
         const V3T<R> n1 = cross3(b1, b2), n2 = cross3(b2, b3);
         const R b2n = r_sqrt<R>(dot3(b2, b2));
         const R phi = r_atan2<R>(b2n * dot3(b1, n2), dot3(n1, n2));
@@ -1500,7 +1551,8 @@ __device__ inline RowType row_type(const float* __restrict__ t) {
 // (1/r is left in *ir_out when the kinds need it, else 0.)
 // Open Ashbaugh-Hatch groups take s^12 - s^6 and r - rsw from rounded s^12 and
 // r; the periodic loop's fused forms round once less.  Each kind of boundary
-// keeps the rounding its trajectories have always had (open_lj).
+// keeps the rounding its trajectories have always had (OPEN_LJ, a template
+// argument: merged as a run-time choice, both would round).
 __device__ __forceinline__ float sub_rounded(float a, float b) {
 #pragma clang fp contract(off)
     return a - b;
@@ -1508,9 +1560,10 @@ __device__ __forceinline__ float sub_rounded(float a, float b) {
 __device__ __forceinline__ bool pair_force_has_ir(int kinds, bool lsw) {
     return (kinds & (kDh | kIsolf)) || ((kinds & (kLja | kUlja)) && lsw);
 }
+template <bool OPEN_LJ = false>
 __device__ __forceinline__ float pair_force(int kinds, bool shared, bool lsw, const PairK<float>& G,
                                             const RowType& ti, const float* __restrict__ tj, float r2,
-                                            float* ir_out = nullptr, bool open_lj = false) {
+                                            float* ir_out = nullptr) {
     const float ir2 = __builtin_amdgcn_rcpf(r2);
     float f = 0.f, r = 0.f, ir = 0.f;
     if (pair_force_has_ir(kinds, lsw)) {
@@ -1541,11 +1594,17 @@ __device__ __forceinline__ float pair_force(int kinds, bool shared, bool lsw, co
         const float er = ti.er + lj.x, ea = ti.ea + lj.z;
         const bool inner = th2 - r2 >= 0.f, outer = r2 - th2 >= 0.f;
         f += inner ? er * X : 0.f;
-        float u = outer ? 4.f * ea * (open_lj ? sub_rounded(s12, s6) : s12 - s6) : 0.f;
+        float s_diff;
+        if constexpr (OPEN_LJ) s_diff = sub_rounded(s12, s6);
+        else s_diff = s12 - s6;
+        float u = outer ? 4.f * ea * s_diff : 0.f;
         float du = outer ? ea * X : 0.f;
         u = inner ? u - ea : u;
         if (lsw) {
-            const float x = fmaxf((open_lj ? sub_rounded(r, G.lja_rsw) : r - G.lja_rsw) * G.lja_inv_sw, 0.f);
+            float r_in;
+            if constexpr (OPEN_LJ) r_in = sub_rounded(r, G.lja_rsw);
+            else r_in = r - G.lja_rsw;
+            const float x = fmaxf(r_in * G.lja_inv_sw, 0.f);
             const float x2 = x * x, x3 = x2 * x;
             const float S = 1.f - x3 * (10.f - 15.f * x + 6.f * x2);
             const float dS = -30.f * x2 * (1.f - x) * (1.f - x) * G.lja_inv_sw;
@@ -1737,7 +1796,7 @@ __device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const 
     float f, ir = 0.f;
     if (SPEC == kSpecExvPeriodic || SPEC == kSpecExvOpen) f = pair_force(kExv, false, false, Kf, rt, tfj, r2f);
     else if (spec_dh(SPEC)) f = pair_force(kDh, false, false, Kf, rt, tfj, r2f, &ir);
-    else if (spec_lj(SPEC)) f = pair_force(kLjr | kLja, true, true, Kf, rt, tfj, r2f, &ir, SPEC == kSpecLjSharedOpen);
+    else if (spec_lj(SPEC)) f = pair_force<SPEC == kSpecLjSharedOpen>(kLjr | kLja, true, true, Kf, rt, tfj, r2f, &ir);
     else if (SPEC == kSpecSolo) f = pair_force(kinds & ~(kExv | kDh | kLjr | kLja), false, Kf.lja_switch, Kf, rt,
                                                tfj, r2f);
     else f = pair_force(kinds & (kExv | kDh | kLjr | kLja), Kf.lj_shared, Kf.lja_switch, Kf, rt, tfj, r2f);
@@ -2208,7 +2267,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pair_energy(
 struct ResArgs {
     const ResSys* tab;
     const ResGroup* grp;
-    const BTerm* terms;        // bead indices local to their system
+    const BTerm* terms;        // bead indices local to their system, times 3
     const float* rows;         // FP32 type rows, kTypeStride floats each
     const DevSys* sys;
     const DevPairGroup* groups;
@@ -2232,6 +2291,8 @@ struct ResArgs {
     int list_cap;              // list entries kept in LDS per system
     const int* excl_tab;       // the groups' exclusion tables (ResGroup::exo), by system
     int ex_cap;                // their LDS words per system
+    const uint32_t* units;     // the units of the bonded terms, by system
+    int unit_cap;              // their LDS words per system
 };
 
 // A pair group's constants, staged in LDS for the whole chunk.
@@ -2248,43 +2309,44 @@ struct ResGroupK {
 
 __host__ __device__ constexpr size_t res_align16(size_t v) { return (v + 15) & ~static_cast<size_t>(15); }
 
-// LDS layout: x, y, z (doubles), f (3 nbs force words; the build's FP32
+// LDS layout: positions (3 nbs doubles), f (3 nbs force words; the build's FP32
 // positions lie over them), the next step's noise (3 nbs floats: gauss3_fast
 // rounds its samples through FP32, so a float holds them exactly), mem and
 // lid (nbs ints each), type rows, group constants, flags, terms, list.
 __host__ __device__ constexpr size_t res_lds_fixed(int nbs) {
     return res_align16(static_cast<size_t>(nbs) * (6 * 8 + 3 * 4 + 2 * 4) +
                        kResMaxTypeRows * kTypeStride * sizeof(float) + kResMaxGroups * sizeof(ResGroupK) +
-                       8 * sizeof(int));
+                       (8 + kResMaxGroups) * sizeof(int));
 }
-__host__ __device__ constexpr size_t res_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap) {
+__host__ __device__ constexpr size_t res_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap, int unit_cap) {
     return res_lds_fixed(nbs) + res_align16(static_cast<size_t>(ex_cap) * sizeof(int)) +
+           res_align16(static_cast<size_t>(unit_cap) * sizeof(uint32_t)) +
            static_cast<size_t>(term_cap) * sizeof(BTerm) + static_cast<size_t>(list_cap) * sizeof(uint32_t);
 }
 
 struct ResLds {
     int nbs;
-    double *x, *y, *z;
-    long long* f;      // fx [0, nbs), fy [nbs, 2 nbs), fz [2 nbs, 3 nbs)
+    double* p;         // positions, x y z of bead b at 3 b: one address per bead, the rest immediate offsets
+    long long* f;      // force words, likewise
     float4* p32;       // the build's FP32 positions, over f (dead while the build runs)
     float* g;          // noise: g0 [0, nbs), g1 [nbs, 2 nbs), g2 [2 nbs, 3 nbs)
     int* mem;          // packed member info of the group being built
     int* lid;          // the beads' indices within their system (noise counters)
     float* rows;
     ResGroupK* gk;
-    int* flag;         // [0] rebuild, [1] FP64 build, [2] entries kept in LDS so far
+    int* flag;         // [0] rebuild, [1] FP64 build, [2] entries kept in LDS so far, [3] where the
+                       // step's units are split, [4] their count, [8 + g] entries of group g
     int* ex;           // the system's exclusion tables
+    uint32_t* unit;    // the units of its bonded terms
     BTerm* terms;
     uint32_t* list;
 };
 
-__device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term_cap, int ex_cap) {
+__device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term_cap, int ex_cap, int unit_cap) {
     ResLds L;
     L.nbs = nbs;
-    L.x = reinterpret_cast<double*>(base);
-    L.y = L.x + nbs;
-    L.z = L.y + nbs;
-    L.f = reinterpret_cast<long long*>(L.z + nbs);
+    L.p = reinterpret_cast<double*>(base);
+    L.f = reinterpret_cast<long long*>(L.p + 3 * nbs);
     L.p32 = reinterpret_cast<float4*>(L.f);
     L.g = reinterpret_cast<float*>(L.f + 3 * nbs);
     L.mem = reinterpret_cast<int*>(L.g + 3 * nbs);
@@ -2293,7 +2355,10 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
     L.gk = reinterpret_cast<ResGroupK*>(L.rows + kResMaxTypeRows * kTypeStride);
     L.flag = reinterpret_cast<int*>(L.gk + kResMaxGroups);
     L.ex = reinterpret_cast<int*>(base + res_lds_fixed(nbs));
-    L.terms = reinterpret_cast<BTerm*>(base + res_lds_fixed(nbs) + res_align16(static_cast<size_t>(ex_cap) * sizeof(int)));
+    L.unit = reinterpret_cast<uint32_t*>(reinterpret_cast<unsigned char*>(L.ex) +
+                                         res_align16(static_cast<size_t>(ex_cap) * sizeof(int)));
+    L.terms = reinterpret_cast<BTerm*>(reinterpret_cast<unsigned char*>(L.unit) +
+                                       res_align16(static_cast<size_t>(unit_cap) * sizeof(uint32_t)));
     L.list = reinterpret_cast<uint32_t*>(L.terms + term_cap);
     return L;
 }
@@ -2315,15 +2380,15 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
     if (tid == 0) { L.flag[1] = 0; L.flag[2] = 0; }
     __syncthreads();
     if (tid < R.nb) {
-        double x = L.x[tid], y = L.y[tid], z = L.z[tid];
+        double x = L.p[3 * tid], y = L.p[3 * tid + 1], z = L.p[3 * tid + 2];
         if (S.periodic) {
             x = wrap_coord(x, S.box[0], S.inv_box[0]);
             y = wrap_coord(y, S.box[1], S.inv_box[1]);
             z = wrap_coord(z, S.box[2], S.inv_box[2]);
         } else {
-            x -= L.x[0];
-            y -= L.y[0];
-            z -= L.z[0];
+            x -= L.p[0];
+            y -= L.p[1];
+            z -= L.p[2];
         }
         L.p32[tid] = make_float4(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z), 0.f);
         if (!(fabs(x) <= kResWide && fabs(y) <= kResWide && fabs(z) <= kResWide)) L.flag[1] = 1;
@@ -2438,7 +2503,8 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
                     const int bi = first ? bia : bib;
                     const int mj = L.mem[j];
                     const int bj = mj & 1023;
-                    double dx = L.x[bj] - L.x[bi], dy = L.y[bj] - L.y[bi], dz = L.z[bj] - L.z[bi];
+                    const double *pi = L.p + 3 * bi, *pj = L.p + 3 * bj;
+                    double dx = pj[0] - pi[0], dy = pj[1] - pi[1], dz = pj[2] - pi[2];
                     if (per) {
                         dx = min_image(dx, G.box[0], G.inv_box[0]);
                         dy = min_image(dy, G.box[1], G.inv_box[1]);
@@ -2459,34 +2525,72 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
             K.lds_off = lds_base;
             K.lds_cnt = min(K.cnt, max(lds_room, 0));
             L.flag[2] = lds_base + K.lds_cnt;
+            L.flag[8 + g] = K.cnt;
         }
         __syncthreads();   // p32 is no longer read; the LDS offset is published
     }
 }
 
-// The first item of the range [off, off + n) of the step's work sequence that
-// thread tid takes (items u with u % T == tid), as an index into the range.
-template <int T>
-__device__ __forceinline__ int res_first(int off) {
-    return static_cast<int>((static_cast<unsigned>(threadIdx.x) - static_cast<unsigned>(off)) % T);
+// A step's work in units of 64 items (one per lane): the bonded terms, a run
+// of one kind after another, costly kinds first, then each pair group's
+// entries, then the next step's noise; a unit never holds two kinds' code.
+// Half of the wavefronts (two of the four on each SIMD) take units from the
+// front of this sequence and half from its back, meeting at `split`, which
+// halves the estimated cost: the front is arithmetic (bonded terms), the back
+// mostly LDS traffic (entries: 20 reads and 6 atomics), and a SIMD that holds
+// both at a time overlaps them.  Everything here is the same for a whole
+// wavefront and sits in scalar registers; a wavefront passes over a group it
+// has no unit of without touching its constants.
+template <int W>
+struct ResDeal {
+    static constexpr int H = W / 2, kNone = 0x40000000;
+    int u, stop;   // the wavefront's next unit, and the end of its half
+    __device__ __forceinline__ ResDeal(int w, int split, int total) {
+        const int k = (w & 3) + 4 * (w >> 3);   // its place among its half
+        const bool back = ((w >> 2) & 1) != 0;
+        u = (back ? split : 0) + k;
+        stop = back ? total : split;
+        if (u >= stop) u = kNone;
+    }
+    __device__ __forceinline__ void next() {
+        u += H;
+        if (u >= stop) u = kNone;
+    }
+};
+
+// Estimated costs of a unit of entries or noise, in the units of kResUnitCost.
+constexpr int kResPairCost = 10, kResNoiseCost = 9;
+
+// The unit count of the step's sequence and where its cost halves.
+__device__ inline void res_split(const ResSys& R, const ResLds& L) {
+    int total = R.ucost + ((R.nb + 63) >> 6) * kResNoiseCost, units = R.nu + ((R.nb + 63) >> 6);
+    for (int g = 0; g < R.ng; ++g) {
+        const int nu = (L.flag[8 + g] + 63) >> 6;
+        total += nu * kResPairCost;
+        units += nu;
+    }
+    int u = R.nu, sum = R.ucost;
+    if (2 * sum >= total)
+        while (u > 0 && 2 * (sum - static_cast<int>(L.unit[u - 1] >> 26)) >= total) sum -= static_cast<int>(L.unit[--u] >> 26);
+    else
+        u = min(units, u + ((total + 1) / 2 - sum + kResPairCost - 1) / kResPairCost);
+    L.flag[3] = u;
+    L.flag[4] = units;
 }
 
 template <int SPEC, int T>
-__device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, int off, const ResLds& L, int& bad) {
-    // a thread with no entry of this group reads none of its constants
-    const int e0 = res_first<T>(off);
-    if (e0 >= K.cnt) return;
+__device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, int beg, int end, int cnt,
+                                          ResDeal<T / 64>& D, const ResLds& L, int& bad) {
     const uint32_t* glist = a.list + K.l0;
     const uint32_t* llist = L.list + K.lds_off;
-    const int cnt = K.cnt, lcnt = K.lds_cnt;
+    const int lcnt = K.lds_cnt;
     const RowGeom geo = K.geo;
     const PairK<float> Kf = K.Kf;
     const int kinds = K.kinds;
-    const int nbs = L.nbs;
-    unsigned long long* F = reinterpret_cast<unsigned long long*>(L.f);
     auto entry = [&](uint32_t w) {
-        const int bi = w & 1023, bj = (w >> 10) & 1023, ti = (w >> 20) & 63, tj = w >> 26;
-        double dx = L.x[bj] - L.x[bi], dy = L.y[bj] - L.y[bi], dz = L.z[bj] - L.z[bi];
+        const int bi = 3 * (w & 1023), bj = 3 * ((w >> 10) & 1023), ti = (w >> 20) & 63, tj = w >> 26;
+        const double *pi = L.p + bi, *pj = L.p + bj;
+        double dx = pj[0] - pi[0], dy = pj[1] - pi[1], dz = pj[2] - pi[2];
         const RowType rt = row_type(L.rows + ti * kTypeStride);
         const double gs = pair_entry<SPEC>(geo, kinds, Kf, rt, L.rows + tj * kTypeStride, true, dx, dy, dz, bad);
         const unsigned long long cx =
@@ -2495,19 +2599,23 @@ __device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, 
             static_cast<unsigned long long>(__double_as_longlong(fma(gs, dy, kFixMagic))) - kFixMagicBits;
         const unsigned long long cz =
             static_cast<unsigned long long>(__double_as_longlong(fma(gs, dz, kFixMagic))) - kFixMagicBits;
-        atomicAdd(F + bi, cx);
-        atomicAdd(F + nbs + bi, cy);
-        atomicAdd(F + 2 * nbs + bi, cz);
-        atomicAdd(F + bj, 0ull - cx);
-        atomicAdd(F + nbs + bj, 0ull - cy);
-        atomicAdd(F + 2 * nbs + bj, 0ull - cz);
+        unsigned long long* Fi = reinterpret_cast<unsigned long long*>(L.f) + bi;
+        unsigned long long* Fj = reinterpret_cast<unsigned long long*>(L.f) + bj;
+        atomicAdd(Fi, cx);
+        atomicAdd(Fi + 1, cy);
+        atomicAdd(Fi + 2, cz);
+        atomicAdd(Fj, 0ull - cx);
+        atomicAdd(Fj + 1, 0ull - cy);
+        atomicAdd(Fj + 2, 0ull - cz);
     };
     // entries kept in LDS, the rest read through a buffer resource over the
     // group's global region (a different load than LDS's, so neither becomes
     // a generic load, and the entry body is inlined once)
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint32_t*>(glist), 0, cnt * static_cast<int>(sizeof(uint32_t)), 0x00020000);
-    for (int e = e0; e < cnt; e += T) {
+    for (; D.u < end; D.next()) {
+        const int e = (D.u - beg) * 64 + static_cast<int>(threadIdx.x & 63u);
+        if (e >= cnt) continue;
         uint32_t w;
         if (e < lcnt) w = llist[e];
         else w = static_cast<uint32_t>(__builtin_amdgcn_raw_buffer_load_b32(grs, e * 4, 0, 0));
@@ -2516,36 +2624,26 @@ __device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, 
 }
 
 // The force pass, and (noise != 0) every bead's noise for global step
-// `nstep`: the sequence terms, list entries group by group, beads.
+// `nstep`.
 template <int T>
 __device__ __forceinline__ void res_forces(const ResArgs& a, const ResSys& R, const DevSys& S, const ResLds& L,
                                            int noise, long long nstep, int& bad) {
-    const ForceOut out{L.f, L.f + L.nbs, L.f + 2 * L.nbs};
+    const ForceOut out{L.f, L.f + 1, L.f + 2};   // the terms hold 3 x bead indices
     const int nl = min(R.nt, a.term_cap);
+    const int lane = static_cast<int>(threadIdx.x & 63u);
+    ResDeal<T / 64> D(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)),
+                      __builtin_amdgcn_readfirstlane(L.flag[3]), __builtin_amdgcn_readfirstlane(L.flag[4]));
     // terms past term_cap through a buffer resource (as the list entries)
     static_assert(sizeof(BTerm) == 48, "a term is three 16-byte loads");
     const __amdgpu_buffer_rsrc_t trs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<BTerm*>(a.terms + R.t0), 0, R.nt * static_cast<int>(sizeof(BTerm)), 0x00020000);
-    // Each run of one bonded kind, and each pair group below, starts its
-    // share of the work on a wavefront boundary (the work sequence is padded
-    // to multiples of 64), so no wavefront runs two kinds' code one after the
-    // other.  A slot finds its run by an unrolled walk over the run table,
-    // which the system record holds in scalar registers (a loop indexing it
-    // would load it from memory once per run and step).
-    int off = 0;
-#pragma unroll
-    for (int q = 0; q < kResMaxSeg; ++q)
-        if (q < R.nseg) off += (R.seg_n[q] + 63) & ~63;
-    for (int v = threadIdx.x; v < off; v += T) {
-        int t = -1, base = 0;
-#pragma unroll
-        for (int q = 0; q < kResMaxSeg; ++q) {
-            if (q < R.nseg) {
-                if (v >= base && v < base + R.seg_n[q]) t = R.seg_t[q] + (v - base);
-                base += (R.seg_n[q] + 63) & ~63;
-            }
-        }
-        if (t < 0) continue;   // padding of a run
+    int end = R.nu;
+    for (; D.u < end; D.next()) {
+        // {first term, terms - 1, cost} of the unit
+        const uint32_t w0 = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(L.unit[D.u])));
+        const int first = static_cast<int>(w0 & 0xFFFFFu), n = static_cast<int>((w0 >> 20) & 63u) + 1;
+        if (lane >= n) continue;   // padding of a run
+        const int t = first + lane;
         BTerm tm;
         if (t < nl) {
             tm = L.terms[t];
@@ -2558,24 +2656,32 @@ __device__ __forceinline__ void res_forces(const ResArgs& a, const ResSys& R, co
             }
             __builtin_memcpy(&tm, w, sizeof(tm));
         }
-        bonded_term<false, float>(tm, S, L.x, L.y, L.z, a.fla, a.fld, out, nullptr, R.sys, bad);
+        bonded_term<false, float>(tm, S, L.p, L.p + 1, L.p + 2, a.fla, a.fld, out, nullptr, R.sys, bad);
     }
+    if (D.u >= ResDeal<T / 64>::kNone) return;   // nothing left for this wavefront
     for (int g = 0; g < R.ng; ++g) {
+        const int cnt = __builtin_amdgcn_readfirstlane(L.flag[8 + g]);
+        const int beg = end;
+        end += (cnt + 63) >> 6;
+        if (D.u >= end) continue;
         const ResGroupK& K = L.gk[g];
         switch (K.spec) {
-        case kSpecExvPeriodic: res_pairs<kSpecExvPeriodic, T>(a, K, off, L, bad); break;
-        case kSpecExvOpen: res_pairs<kSpecExvOpen, T>(a, K, off, L, bad); break;
-        case kSpecDh: res_pairs<kSpecDh, T>(a, K, off, L, bad); break;
-        case kSpecLjShared: res_pairs<kSpecLjShared, T>(a, K, off, L, bad); break;
-        case kSpecDhOpen: res_pairs<kSpecDhOpen, T>(a, K, off, L, bad); break;
-        case kSpecLjSharedOpen: res_pairs<kSpecLjSharedOpen, T>(a, K, off, L, bad); break;
-        case kSpecSolo: res_pairs<kSpecSolo, T>(a, K, off, L, bad); break;
-        default: res_pairs<kSpecGeneric, T>(a, K, off, L, bad); break;
+        case kSpecExvPeriodic: res_pairs<kSpecExvPeriodic, T>(a, K, beg, end, cnt, D, L, bad); break;
+        case kSpecExvOpen: res_pairs<kSpecExvOpen, T>(a, K, beg, end, cnt, D, L, bad); break;
+        case kSpecDh: res_pairs<kSpecDh, T>(a, K, beg, end, cnt, D, L, bad); break;
+        case kSpecLjShared: res_pairs<kSpecLjShared, T>(a, K, beg, end, cnt, D, L, bad); break;
+        case kSpecDhOpen: res_pairs<kSpecDhOpen, T>(a, K, beg, end, cnt, D, L, bad); break;
+        case kSpecLjSharedOpen: res_pairs<kSpecLjSharedOpen, T>(a, K, beg, end, cnt, D, L, bad); break;
+        case kSpecSolo: res_pairs<kSpecSolo, T>(a, K, beg, end, cnt, D, L, bad); break;
+        default: res_pairs<kSpecGeneric, T>(a, K, beg, end, cnt, D, L, bad); break;
         }
-        off += (K.cnt + 63) & ~63;
     }
     if (noise) {
-        for (int b = res_first<T>(off); b < R.nb; b += T) {
+        const int beg = end;
+        end += (R.nb + 63) >> 6;
+        for (; D.u < end; D.next()) {
+            const int b = (D.u - beg) * 64 + lane;
+            if (b >= R.nb) continue;
             double g[3];
             gauss3_fast(S.seed, static_cast<uint64_t>(nstep - S.step_origin), static_cast<uint32_t>(L.lid[b]), g);
             L.g[b] = static_cast<float>(g[0]);
@@ -2593,7 +2699,7 @@ __device__ __forceinline__ void res_forces(const ResArgs& a, const ResSys& R, co
 template <int T>
 __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char res_base[];
-    const ResLds L = res_lds(res_base, a.nbs, a.term_cap, a.ex_cap);
+    const ResLds L = res_lds(res_base, a.nbs, a.term_cap, a.ex_cap, a.unit_cap);
     const ResSys R = a.tab[blockIdx.x];
     const DevSys S = a.sys[R.sys];
     const int tid = threadIdx.x;
@@ -2601,15 +2707,16 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
     const bool own = tid < R.nb;
     const int gb = R.b0 + tid;
     double X[3] = {0, 0, 0}, V[3] = {0, 0, 0}, ref[3] = {0, 0, 0};
-    double im = 0.0, hs2 = 0.0;
+    double im = 0.0, hs2 = 0.0, sig = 0.0;
     int bad = 0;
     const long long step0 = a.gstep[0];
     if (own) {
         X[0] = a.px[gb]; X[1] = a.py[gb]; X[2] = a.pz[gb];
         V[0] = a.vx[gb]; V[1] = a.vy[gb]; V[2] = a.vz[gb];
         im = a.inv_m[gb];
+        sig = noise_sigma(S, im);   // kept for the launch
         hs2 = a.bead_hs2[gb];
-        L.x[tid] = X[0]; L.y[tid] = X[1]; L.z[tid] = X[2];
+        L.p[3 * tid] = X[0]; L.p[3 * tid + 1] = X[1]; L.p[3 * tid + 2] = X[2];
         const int lid = a.local_id[gb];
         L.lid[tid] = lid;
         double g[3];
@@ -2627,6 +2734,7 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         for (int k = tid; k < nw; k += T) dst[k] = src[k];
     }
     for (int k = tid; k < R.exn; k += T) L.ex[k] = a.excl_tab[R.ex0 + k];
+    for (int k = tid; k < R.nu; k += T) L.unit[k] = a.units[R.u0 + k];
     if (tid < R.ng) {
         const ResGroup Q = a.grp[R.g0 + tid];
         const DevPairGroup& G = a.groups[Q.gid];
@@ -2648,40 +2756,42 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         K.cnt = 0;
         K.rl2w = Q.rl2w;
     }
-    if (tid == 0) L.flag[0] = 0;
+    if (tid < 8 + kResMaxGroups) L.flag[tid] = 0;
     __syncthreads();
     res_build<T>(a, R, S, L);
+    if (tid == 0) res_split(a.tab[blockIdx.x], L);
     ref[0] = X[0]; ref[1] = X[1]; ref[2] = X[2];
     if (own) {
-        L.f[tid] = a.fx[gb];
-        L.f[nbs + tid] = a.fy[gb];
-        L.f[2 * nbs + tid] = a.fz[gb];
+        L.f[3 * tid] = a.fx[gb];
+        L.f[3 * tid + 1] = a.fy[gb];
+        L.f[3 * tid + 2] = a.fz[gb];
     }
     __syncthreads();
     for (int s = 0; s < a.nsteps; ++s) {
         if (own) {
-            const long long F0 = L.f[tid], F1 = L.f[nbs + tid], F2 = L.f[2 * nbs + tid];
-            L.f[tid] = 0;   // read: the force pass after the barrier refills them
-            L.f[nbs + tid] = 0;
-            L.f[2 * nbs + tid] = 0;
+            const long long F0 = L.f[3 * tid], F1 = L.f[3 * tid + 1], F2 = L.f[3 * tid + 2];
+            L.f[3 * tid] = 0;   // read: the force pass after the barrier refills them
+            L.f[3 * tid + 1] = 0;
+            L.f[3 * tid + 2] = 0;
             const double g[3] = {L.g[tid], L.g[nbs + tid], L.g[2 * nbs + tid]};
             double xn[3], vn[3];
-            if (!baoab_bead_g(S, im, F0, F1, F2, X, V, s > 0 ? 1 : 0, g, xn, vn)) bad = 1;
+            if (!baoab_bead_g(S, im, sig, F0, F1, F2, X, V, s > 0 ? 1 : 0, g, xn, vn)) bad = 1;
             X[0] = xn[0]; X[1] = xn[1]; X[2] = xn[2];
             V[0] = vn[0]; V[1] = vn[1]; V[2] = vn[2];
-            L.x[tid] = X[0]; L.y[tid] = X[1]; L.z[tid] = X[2];
+            L.p[3 * tid] = X[0]; L.p[3 * tid + 1] = X[1]; L.p[3 * tid + 2] = X[2];
             const double dx = X[0] - ref[0], dy = X[1] - ref[1], dz = X[2] - ref[2];
             if (!(dist2(dx, dy, dz) <= hs2)) L.flag[0] = 1;
         }
         __syncthreads();
         if (L.flag[0] != 0) {   // uniform: every thread reads it after the barrier
             res_build<T>(a, R, S, L);
+            if (tid == 0) res_split(a.tab[blockIdx.x], L);
             ref[0] = X[0]; ref[1] = X[1]; ref[2] = X[2];
             if (tid == 0) L.flag[0] = 0;   // read by all before the build's barriers
             if (own) {   // the build's FP32 positions lay over the force words
-                L.f[tid] = 0;
-                L.f[nbs + tid] = 0;
-                L.f[2 * nbs + tid] = 0;
+                L.f[3 * tid] = 0;
+                L.f[3 * tid + 1] = 0;
+                L.f[3 * tid + 2] = 0;
             }
             __syncthreads();
         }
@@ -2690,7 +2800,7 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         __syncthreads();
     }
     if (own) {
-        const long long F0 = L.f[tid], F1 = L.f[nbs + tid], F2 = L.f[2 * nbs + tid];
+        const long long F0 = L.f[3 * tid], F1 = L.f[3 * tid + 1], F2 = L.f[3 * tid + 2];
         if (im != 0.0) {   // the closing half kick, as k_half_kick
             V[0] = half_kick(V[0], S.half_dt, F0 * kFixInv, im);
             V[1] = half_kick(V[1], S.half_dt, F1 * kFixInv, im);
@@ -3041,15 +3151,12 @@ void launch_pair(const DevPtrs& d, hipStream_t st, bool energy, const ForceBuf& 
 
 int pair_grid_size(const DevPtrs& d) { return std::min(d.n_pair_blocks, d.pair_grid); }
 
-size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap) {
-    return res_lds_bytes(nbs, term_cap, list_cap, ex_cap);
+size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap, int unit_cap) {
+    return res_lds_bytes(nbs, term_cap, list_cap, ex_cap, unit_cap);
 }
 
-hipError_t resident_prepare(int threads, size_t lds) {
-    const void* f = threads == 256 ? reinterpret_cast<const void*>(&k_resident<256>)
-                  : threads == 512 ? reinterpret_cast<const void*>(&k_resident<512>)
-                                   : reinterpret_cast<const void*>(&k_resident<1024>);
-    return hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+hipError_t resident_prepare(size_t lds) {
+    return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_resident<kResThreads>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
 }
 
 void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host) {
@@ -3057,13 +3164,10 @@ void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host) {
     const ResArgs a{d.res_tab, d.res_grp, d.res_terms, d.res_rows, d.sys, d.groups, d.member_bead, d.member_type,
                     d.local_id, d.inv_m, d.res_hs2, d.px, d.py, d.pz,
                     d.vx, d.vy, d.vz, d.f.fx, d.f.fy, d.f.fz, d.res_list, d.fla, d.fld, d.gstep, d.err,
-                    d.flags, host, nsteps, d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_excl, d.res_ex_cap};
-    const size_t lds = res_lds_bytes(d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_ex_cap);
-    switch (d.res_threads) {
-    case 256: k_resident<256><<<d.res_n, 256, lds, st>>>(a); break;
-    case 512: k_resident<512><<<d.res_n, 512, lds, st>>>(a); break;
-    default: k_resident<1024><<<d.res_n, 1024, lds, st>>>(a); break;
-    }
+                    d.flags, host, nsteps, d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_excl, d.res_ex_cap,
+                    d.res_units, d.res_unit_cap};
+    const size_t lds = res_lds_bytes(d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_ex_cap, d.res_unit_cap);
+    k_resident<kResThreads><<<d.res_n, kResThreads, lds, st>>>(a);
     if (d.res_n > 1) launch_status_out(d, st, host, nsteps);
 }
 

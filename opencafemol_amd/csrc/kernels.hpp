@@ -83,6 +83,8 @@ struct DevPtrs {
     int res_nbs = 0;                          // LDS entries per bead array (multiple of 64)
     int res_ex_cap = 0;                       // exclusion-table words per system (staged in LDS)
     int* res_excl = nullptr;
+    int res_unit_cap = 0;                     // words of a system's unit table (staged in LDS)
+    uint32_t* res_units = nullptr;
     double* res_hs2 = nullptr;                // per bead: (resident skin / 2)^2
     ResSys* res_tab = nullptr;
     ResGroup* res_grp = nullptr;
@@ -155,8 +157,10 @@ int pair_grid_size(const DevPtrs& d);
 void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host);
 // LDS of one resident workgroup (bead arrays of nbs entries), and the
 // attribute that allows it (gfx950 gives a workgroup up to 160 KB).
-size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap);
-hipError_t resident_prepare(int threads, size_t lds);
+size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap, int unit_cap);
+hipError_t resident_prepare(size_t lds);
+// One workgroup size: a step's units are dealt over all of its wavefronts.
+constexpr int kResThreads = 1024;
 constexpr size_t kResLdsMax = 160 * 1024;
 void launch_reduce_stamps(hipStream_t st, const unsigned long long* stamp, int nlaunch, int nblk,
                           unsigned long long* out);

@@ -1,0 +1,66 @@
+"""Resident steps around the sizes where the step's units of 64 items change:
+chains whose term counts fill a unit exactly, miss it or pass it by one, and
+systems with bonded terms only, pairs only or neither.  The standard path is
+the reference; both sum the same fixed-point words, so the states are equal
+bit for bit (no tolerance)."""
+import sys
+
+import numpy as np
+import pytest
+
+from opencafemol_amd import abi, configs
+from opencafemol_amd.context import Context
+from opencafemol_amd.model import SystemSpec
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def _announce(request):
+    sys.__stderr__.write(f"\n[gpu-case] {request.node.nodeid}\n")
+    sys.__stderr__.flush()
+    yield
+
+
+def _both(s, it, x, steps):
+    v = np.random.default_rng(1).normal(scale=0.1, size=x.shape)
+    got = []
+    for resident in (-1, 0):
+        with Context(s, it, resident=resident) as c:
+            assert (c.resident_threads() > 0) == (resident != 0)
+            c.set_positions(x)
+            c.set_velocities(v)
+            assert c.step(steps) == 0
+            st = c.get_state(abi.STATE_POSITIONS | abi.STATE_VELOCITIES | abi.STATE_FORCES)
+            got.append((st["positions"], st["velocities"], st["forces"], st["step"]))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n", [5, 64, 65, 66, 67, 68, 129, 130, 131, 450, 1024])
+def test_go_chain_unit_edges(n):
+    s, it, x = configs.go_chain(n, seed=n)
+    _both(s, it, x, 60)
+
+
+def _only(s, keep):
+    out = SystemSpec(masses=s.masses, box=s.box)
+    for f in s.forces:
+        if keep(f):
+            out.add(f)
+    return out
+
+
+@pytest.mark.parametrize("what", ["bonded", "pairs", "none", "one pair group"])
+def test_partial_sequences(what):
+    s, it, x = configs.go_chain(70, seed=4)
+    keep = {"bonded": lambda f: f.kind < abi.EXCLUDED_VOLUME, "pairs": lambda f: f.kind >= abi.EXCLUDED_VOLUME,
+            "none": lambda f: False, "one pair group": lambda f: f.kind == abi.DEBYE_HUCKEL}[what]
+    _both(_only(s, keep), it, x, 40)
+
+
+def test_open_hps_chain():
+    """Open Ashbaugh-Hatch and Debye-Hueckel groups (their own row loops)."""
+    s, it, x = configs.hps_open_cluster(6, 100, extent=(5.0, 5.0), seed=2)
+    x = x + np.random.default_rng(0).normal(scale=0.005, size=x.shape)
+    _both(s, it, x, 5)
