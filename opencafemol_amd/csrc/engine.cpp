@@ -877,17 +877,17 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
                 rexcl.push_back(at);
                 for (int i = 0; i < Q.nm; ++i) rexcl.insert(rexcl.end(), far[i].begin(), far[i].end());
             }
-            // the resident list's skin: at most kResSkin (a list read every
-            // step by one workgroup pays for its width at every step, a
-            // rebuild is cheap); the FP32 test's threshold adds 1e-3 nm, well
-            // above the 2.2e-4 nm error of coordinates below kResWide
-            const double skin_r = std::min(2.0 * std::sqrt(G.half_skin2), kResSkin);
-            const double rl = G.rc + skin_r;
-            Q.rl2 = rl * rl;
-            Q.rl2w = static_cast<float>((rl + 1e-3) * (rl + 1e-3));
+            // the FP32 thresholds add 1e-3 nm, well above the 2.2e-4 nm error
+            // of coordinates below kResWide
+            const double skin = 2.0 * std::sqrt(G.half_skin2);
+            const double skin_w = std::min(skin, kResSkinPruned), skin_n = std::min(skin, kResSkin);
+            Q.rl2 = (G.rc + skin_w) * (G.rc + skin_w);
+            Q.rl2s = (G.rc + skin_n) * (G.rc + skin_n);
+            Q.rl2w = static_cast<float>((G.rc + skin_w + 1e-3) * (G.rc + skin_w + 1e-3));
+            Q.rl2ws = static_cast<float>((G.rc + skin_n + 1e-3) * (G.rc + skin_n + 1e-3));
             for (int i = 0; i < G.member_count; ++i) {
                 double& h = res_hs2[excl_bead_[G.member_begin + i]];
-                h = std::min(h, 0.25 * skin_r * skin_r);
+                h = std::min(h, 0.25 * skin_w * skin_w);
             }
             l0 += std::max<long long>(1, static_cast<long long>(Q.nm) * (Q.nm - 1) / 2);
             for (int k = 0; k < G.n_types * kTypeStride; ++k)
@@ -930,10 +930,14 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     const size_t fixed = resident_lds_bytes(d_.res_nbs, 0, 0, d_.res_ex_cap, d_.res_unit_cap);
     if (fixed > budget) { d_.res_n = 0; return; }
     const size_t room = budget - fixed;
-    d_.res_list_cap = static_cast<int>(std::min<long long>({max_pairs, kResListLdsMax,
-                                                            static_cast<long long>(room / sizeof(uint32_t))}));
+    // half of the list's LDS first, then the terms, then the rest of the list
+    const auto list_for = [&](long long most, size_t bytes) {
+        return static_cast<int>(std::min<long long>({max_pairs, most, static_cast<long long>(bytes / sizeof(uint32_t))}));
+    };
+    const int list_first = list_for(kResListLdsMax / 2, room);
     d_.res_term_cap = static_cast<int>(std::min<size_t>(static_cast<size_t>(max_nt),
-                                                        (room - d_.res_list_cap * sizeof(uint32_t)) / sizeof(BTerm)));
+                                                        (room - list_first * sizeof(uint32_t)) / sizeof(BTerm)));
+    d_.res_list_cap = list_for(kResListLdsMax, room - d_.res_term_cap * sizeof(BTerm));
     const size_t lds = resident_lds_bytes(d_.res_nbs, d_.res_term_cap, d_.res_list_cap, d_.res_ex_cap, d_.res_unit_cap);
     check_hip(resident_prepare(lds), "hipFuncSetAttribute (resident LDS)");
     d_.res_tab = dalloc<ResSys>(tab.size()); upload(d_.res_tab, tab);
@@ -950,6 +954,7 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     if (!rexcl.empty()) upload(d_.res_excl, rexcl);
     d_.res_units = dalloc<uint32_t>(std::max<size_t>(units.size(), 1));
     if (!units.empty()) upload(d_.res_units, units);
+    d_.prune_hm2 = prune_hm2_;
     d_.res_n = nsys;
 }
 

@@ -2293,6 +2293,7 @@ struct ResArgs {
     int ex_cap;                // their LDS words per system
     const uint32_t* units;     // the units of the bonded terms, by system
     int unit_cap;              // their LDS words per system
+    double prune_hm2;          // (margin / 2)^2, slightly reduced
 };
 
 // A pair group's constants, staged in LDS for the whole chunk.
@@ -2300,21 +2301,22 @@ struct ResGroupK {
     RowGeom geo;
     PairK<float> Kf;
     long long l0;      // list region in global memory
-    double rl2;             // (cutoff + resident skin)^2
+    double rl2, rl2s;       // (cutoff + resident skin)^2 with the wide and the narrow skin
     int kinds, spec, m0, nm, trow, gid, exo;
     int lds_off, lds_cnt;   // the group's entries kept in LDS: [lds_off, lds_off + lds_cnt)
-    int cnt;                // entries of the last build
-    float rl2w;
+    int ocnt;               // entries of the last build, in the group's global region
+    int cnt;                // entries the force pass reads
+    float rl2w, rl2ws;
 };
 
 __host__ __device__ constexpr size_t res_align16(size_t v) { return (v + 15) & ~static_cast<size_t>(15); }
 
 // LDS layout: positions (3 nbs doubles), f (3 nbs force words; the build's FP32
-// positions lie over them), the next step's noise (3 nbs floats: gauss3_fast
-// rounds its samples through FP32, so a float holds them exactly), mem and
-// lid (nbs ints each), type rows, group constants, flags, terms, list.
+// positions lie over them), the last build's positions, the next step's noise (3 nbs floats: gauss3_fast
+// rounds its samples through FP32, so a float holds them exactly), pr (3 nbs
+// floats), mem and lid (nbs ints each), type rows, group constants, flags, terms, list.
 __host__ __device__ constexpr size_t res_lds_fixed(int nbs) {
-    return res_align16(static_cast<size_t>(nbs) * (6 * 8 + 3 * 4 + 2 * 4) +
+    return res_align16(static_cast<size_t>(nbs) * (9 * 8 + 3 * 4 + 3 * 4 + 2 * 4) +
                        kResMaxTypeRows * kTypeStride * sizeof(float) + kResMaxGroups * sizeof(ResGroupK) +
                        (8 + kResMaxGroups) * sizeof(int));
 }
@@ -2328,14 +2330,17 @@ struct ResLds {
     int nbs;
     double* p;         // positions, x y z of bead b at 3 b: one address per bead, the rest immediate offsets
     long long* f;      // force words, likewise
+    double* ref;       // positions at the last build, likewise
     float4* p32;       // the build's FP32 positions, over f (dead while the build runs)
     float* g;          // noise: g0 [0, nbs), g1 [nbs, 2 nbs), g2 [2 nbs, 3 nbs)
+    float* pr;         // displacements from the build's positions at the last prune, x y z at 3 b
     int* mem;          // packed member info of the group being built
     int* lid;          // the beads' indices within their system (noise counters)
     float* rows;
     ResGroupK* gk;
-    int* flag;         // [0] rebuild, [1] FP64 build, [2] entries kept in LDS so far, [3] where the
-                       // step's units are split, [4] their count, [8 + g] entries of group g
+    int* flag;         // [0] rebuild, [1] FP64 build, [3] where the
+                       // step's units are split, [4] their count, [5] prune, [6] the pruned lists
+                       // did not fit, [8 + g] entries of group g
     int* ex;           // the system's exclusion tables
     uint32_t* unit;    // the units of its bonded terms
     BTerm* terms;
@@ -2348,8 +2353,10 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
     L.p = reinterpret_cast<double*>(base);
     L.f = reinterpret_cast<long long*>(L.p + 3 * nbs);
     L.p32 = reinterpret_cast<float4*>(L.f);
-    L.g = reinterpret_cast<float*>(L.f + 3 * nbs);
-    L.mem = reinterpret_cast<int*>(L.g + 3 * nbs);
+    L.ref = reinterpret_cast<double*>(L.f + 3 * nbs);
+    L.g = reinterpret_cast<float*>(L.ref + 3 * nbs);
+    L.pr = L.g + 3 * nbs;
+    L.mem = reinterpret_cast<int*>(L.pr + 3 * nbs);
     L.lid = L.mem + nbs;
     L.rows = reinterpret_cast<float*>(L.lid + nbs);
     L.gk = reinterpret_cast<ResGroupK*>(L.rows + kResMaxTypeRows * kTypeStride);
@@ -2363,10 +2370,10 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
     return L;
 }
 
-// Lists of every group of the system at the positions in LDS.  All threads
-// call it; it overwrites the force words (p32 lies over them) and ends with a
-// barrier, after which they may be written again.  Entries go to LDS while
-// the system's list_cap lasts, then to the group's global region.
+// Lists of every group of the system at the positions in LDS, into the groups'
+// global regions, with the wide or the narrow skin.  All threads call it; it
+// overwrites the force words (p32 lies over them) and ends with a barrier,
+// after which they may be written again.
 // The member pairs (i, j > i) are dealt over all threads: rows r and
 // nm - 1 - r together hold nm - 1 candidates, and each such row pair is cut
 // into S segments so that about 2T segments cover the group; a thread tests
@@ -2374,10 +2381,10 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
 // mask bit for the next kResNearExcl members, a search of the short sorted
 // list of farther ones, both in LDS).
 template <int T>
-__device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, const ResLds& L) {
+__device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, const ResLds& L, bool wide_skin) {
     const int tid = threadIdx.x;
     if (R.ng == 0) return;   // uniform; nothing is written
-    if (tid == 0) { L.flag[1] = 0; L.flag[2] = 0; }
+    if (tid == 0) L.flag[1] = 0;
     __syncthreads();
     if (tid < R.nb) {
         double x = L.p[3 * tid], y = L.p[3 * tid + 1], z = L.p[3 * tid + 2];
@@ -2396,7 +2403,7 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
     for (int g = 0; g < R.ng; ++g) {
         ResGroupK& K = L.gk[g];
         const DevPairGroup& G = a.groups[K.gid];
-        if (tid == 0) K.cnt = 0;
+        if (tid == 0) K.ocnt = 0;
         if (tid < K.nm) {
             const int m = K.m0 + tid;
             const int mt = a.member_type[m];
@@ -2406,8 +2413,8 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
         const bool wide = L.flag[1] != 0;
         const bool per = K.geo.periodic;
         const int nm = K.nm;
-        const int lds_base = L.flag[2];
-        const int lds_room = a.list_cap - lds_base;
+        const float rl2w = wide_skin ? K.rl2w : K.rl2ws;
+        const double rl2 = wide_skin ? K.rl2 : K.rl2s;
         uint32_t* glist = a.list + K.l0;
         const float Lx = static_cast<float>(G.box[0]), Ly = static_cast<float>(G.box[1]);
         const float Lz = static_cast<float>(G.box[2]);
@@ -2428,14 +2435,13 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
             if (m == 0ull) return;                         // the same for every active lane
             const int leader = __ffsll(static_cast<long long>(m)) - 1;
             int base = 0;
-            if (lane == leader) base = atomicAdd(&K.cnt, __popcll(m));
+            if (lane == leader) base = atomicAdd(&K.ocnt, __popcll(m));
             base = __shfl(base, leader, 64);
             if (keep) {
                 const int k = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
                                          static_cast<uint32_t>(m >> 32),
                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
-                if (k < lds_room) L.list[lds_base + k] = w;
-                else glist[k] = w;
+                glist[k] = w;
             }
         };
         auto excluded = [&](int i, int j, uint32_t near_mask, int f0, int f1) {
@@ -2484,7 +2490,7 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
                             dz = fmaf(-Lz, rintf(dz * iLz), dz);
                         }
                         const uint32_t allow = first ? alla : allb;
-                        bool keep = qq < q1 && fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < K.rl2w &&
+                        bool keep = qq < q1 && fmaf(dz, dz, fmaf(dy, dy, dx * dx)) < rl2w &&
                                     ((allow >> (mj[k] >> 16)) & 1u);
                         const int i = first ? r : r2, j = first ? r + 1 + qq : qq + 1;
                         if (keep) keep = !excluded(i, j, first ? nma : nmb, first ? f0a : f0b, first ? f1a : f1b);
@@ -2511,7 +2517,7 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
                         dz = min_image(dz, G.box[2], G.inv_box[2]);
                     }
                     const uint32_t allow = first ? alla : allb;
-                    bool keep = dist2(dx, dy, dz) < K.rl2 && ((allow >> (mj >> 16)) & 1u);
+                    bool keep = dist2(dx, dy, dz) < rl2 && ((allow >> (mj >> 16)) & 1u);
                     if (keep) keep = !excluded(i, j, first ? nma : nmb, first ? f0a : f0b, first ? f1a : f1b);
                     const uint32_t w = static_cast<uint32_t>(bi) | (static_cast<uint32_t>(bj) << 10) |
                                        (static_cast<uint32_t>(first ? tia : tib) << 20) |
@@ -2520,15 +2526,82 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
                 }
             }
         }
-        __syncthreads();   // the count is final; the next group reuses mem
-        if (tid == 0) {
-            K.lds_off = lds_base;
-            K.lds_cnt = min(K.cnt, max(lds_room, 0));
-            L.flag[2] = lds_base + K.lds_cnt;
-            L.flag[8 + g] = K.cnt;
-        }
-        __syncthreads();   // p32 is no longer read; the LDS offset is published
+        __syncthreads();   // the count is final; the next group reuses mem, the caller p32's words
     }
+}
+
+// The entries the force pass reads, from the groups' built lists.  prune: the
+// pairs within cutoff + margin at the positions in LDS, into the groups' shares
+// of the LDS list; flag[6] says that some share was too small.  Otherwise (the
+// pruned lists do not fit): every entry, the first ones of each group in LDS
+// and the rest where the build left them.  All threads call it; it ends with a
+// barrier.  A build costs ~125 k cycles on a 500-bead chain and the entries
+// beyond the cutoff as much as those inside, so lists with a wide skin are
+// built every ~100 steps and pruned every few (~5 k cycles): with one list at
+// 0.3 nm the chain read 2,900 entries a step and built every 31.
+template <int T>
+__device__ void res_take(const ResArgs& a, const ResSys& R, const ResLds& L, bool prune) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (R.ng == 0) return;   // uniform
+    if (tid == 0) L.flag[6] = 0;
+    if (tid < R.ng) L.gk[tid].cnt = 0;
+    __syncthreads();
+    long long total = 0;
+    for (int g = 0; g < R.ng; ++g) total += L.gk[g].ocnt;
+    long long before = 0;
+    for (int g = 0; g < R.ng; ++g) {
+        ResGroupK& K = L.gk[g];
+        const int ocnt = K.ocnt;
+        // a share that holds the whole list while all of them fit, else in proportion
+        const int off = static_cast<int>(total <= a.list_cap ? before : before * a.list_cap / total);
+        before += ocnt;
+        const int room = static_cast<int>(total <= a.list_cap ? before : before * a.list_cap / total) - off;
+        const uint32_t* glist = a.list + K.l0;
+        uint32_t* llist = L.list + off;
+        if (prune) {
+            const RowGeom geo = K.geo;
+            for (int e0 = tid; e0 - lane < ocnt; e0 += 4 * T) {   // whole wavefronts
+                uint32_t w[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) w[k] = glist[min(e0 + k * T, ocnt - 1)];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const double *pi = L.p + 3 * (w[k] & 1023), *pj = L.p + 3 * ((w[k] >> 10) & 1023);
+                    double dx = pj[0] - pi[0], dy = pj[1] - pi[1], dz = pj[2] - pi[2];
+                    if (geo.periodic) {
+                        dx = min_image(dx, geo.bx, geo.ibx);
+                        dy = min_image(dy, geo.by, geo.iby);
+                        dz = min_image(dz, geo.bz, geo.ibz);
+                    }
+                    const bool keep = e0 + k * T < ocnt && dist2(dx, dy, dz) < geo.rin2;
+                    const unsigned long long m = __ballot(keep);
+                    if (m == 0ull) continue;   // the same for the wavefront
+                    int base = 0;
+                    if (lane == 0) base = atomicAdd(&K.cnt, __popcll(m));
+                    base = __builtin_amdgcn_readfirstlane(base);
+                    const int at = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                              static_cast<uint32_t>(m >> 32),
+                                              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+                    if (keep && at < room) llist[at] = w[k];
+                }
+            }
+        } else {
+            for (int e = tid; e < min(ocnt, room); e += T) llist[e] = glist[e];
+        }
+        if (tid == 0) {
+            K.lds_off = off;
+            K.lds_cnt = room;   // final below
+        }
+    }
+    __syncthreads();
+    if (tid < R.ng) {
+        ResGroupK& K = L.gk[tid];
+        if (!prune) K.cnt = K.ocnt;
+        if (prune && K.cnt > K.lds_cnt) L.flag[6] = 1;
+        K.lds_cnt = min(K.cnt, K.lds_cnt);
+        L.flag[8 + tid] = K.cnt;
+    }
+    __syncthreads();
 }
 
 // A step's work in units of 64 items (one per lane): the bonded terms, a run
@@ -2706,17 +2779,20 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
     const int nbs = L.nbs;
     const bool own = tid < R.nb;
     const int gb = R.b0 + tid;
-    double X[3] = {0, 0, 0}, V[3] = {0, 0, 0}, ref[3] = {0, 0, 0};
+    // a bead's velocity and constants stay in its thread's registers, all else
+    // in LDS: the force pass needs the other registers
+    double V[3] = {0, 0, 0};
     double im = 0.0, hs2 = 0.0, sig = 0.0;
     int bad = 0;
     const long long step0 = a.gstep[0];
     if (own) {
-        X[0] = a.px[gb]; X[1] = a.py[gb]; X[2] = a.pz[gb];
         V[0] = a.vx[gb]; V[1] = a.vy[gb]; V[2] = a.vz[gb];
         im = a.inv_m[gb];
         sig = noise_sigma(S, im);   // kept for the launch
         hs2 = a.bead_hs2[gb];
-        L.p[3 * tid] = X[0]; L.p[3 * tid + 1] = X[1]; L.p[3 * tid + 2] = X[2];
+        L.p[3 * tid] = L.ref[3 * tid] = a.px[gb];
+        L.p[3 * tid + 1] = L.ref[3 * tid + 1] = a.py[gb];
+        L.p[3 * tid + 2] = L.ref[3 * tid + 2] = a.pz[gb];
         const int lid = a.local_id[gb];
         L.lid[tid] = lid;
         double g[3];
@@ -2725,6 +2801,7 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         L.g[nbs + tid] = static_cast<float>(g[1]);
         L.g[2 * nbs + tid] = static_cast<float>(g[2]);
     }
+    if (own) L.pr[3 * tid] = L.pr[3 * tid + 1] = L.pr[3 * tid + 2] = 0.f;
     for (int k = tid; k < R.nrow * kTypeStride; k += T) L.rows[k] = a.rows[static_cast<size_t>(R.row0) * kTypeStride + k];
     {
         // the system's bonded terms, 12 words each, as far as term_cap holds
@@ -2751,16 +2828,27 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         K.gid = Q.gid;
         K.exo = Q.exo;
         K.rl2 = Q.rl2;
+        K.rl2s = Q.rl2s;
         K.lds_off = 0;
         K.lds_cnt = 0;
+        K.ocnt = 0;
         K.cnt = 0;
         K.rl2w = Q.rl2w;
+        K.rl2ws = Q.rl2ws;
     }
     if (tid < 8 + kResMaxGroups) L.flag[tid] = 0;
     __syncthreads();
-    res_build<T>(a, R, S, L);
-    if (tid == 0) res_split(a.tab[blockIdx.x], L);
-    ref[0] = X[0]; ref[1] = X[1]; ref[2] = X[2];
+    // lists: built wide and pruned, or, once the pruned lists did not fit the
+    // LDS list, built narrow and taken whole; the first step builds.  A small
+    // system's entries are one unit or less for each wavefront whatever the
+    // skin, and pruning only adds to its step (62 beads: 1.73 us a step with
+    // narrow lists, 1.95 pruned; 213 beads: 4.9 and 4.8; 500: 8.6 and 7.1).
+    bool two = R.nb > kResNarrowBeads;   // uniform
+    if (!two) hs2 = fmin(hs2, 0.25 * kResSkin * kResSkin);
+    if (tid == 0) L.flag[0] = 1;
+    // the FP32 displacement is off by less than 1e-7 nm; the margin's square
+    // is reduced by far more
+    const float hm2 = static_cast<float>(a.prune_hm2 * (1.0 - 1e-4));
     if (own) {
         L.f[3 * tid] = a.fx[gb];
         L.f[3 * tid + 1] = a.fy[gb];
@@ -2774,24 +2862,47 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
             L.f[3 * tid + 1] = 0;
             L.f[3 * tid + 2] = 0;
             const double g[3] = {L.g[tid], L.g[nbs + tid], L.g[2 * nbs + tid]};
+            const double X[3] = {L.p[3 * tid], L.p[3 * tid + 1], L.p[3 * tid + 2]};
             double xn[3], vn[3];
             if (!baoab_bead_g(S, im, sig, F0, F1, F2, X, V, s > 0 ? 1 : 0, g, xn, vn)) bad = 1;
-            X[0] = xn[0]; X[1] = xn[1]; X[2] = xn[2];
             V[0] = vn[0]; V[1] = vn[1]; V[2] = vn[2];
-            L.p[3 * tid] = X[0]; L.p[3 * tid + 1] = X[1]; L.p[3 * tid + 2] = X[2];
-            const double dx = X[0] - ref[0], dy = X[1] - ref[1], dz = X[2] - ref[2];
+            L.p[3 * tid] = xn[0]; L.p[3 * tid + 1] = xn[1]; L.p[3 * tid + 2] = xn[2];
+            const double dx = xn[0] - L.ref[3 * tid], dy = xn[1] - L.ref[3 * tid + 1];
+            const double dz = xn[2] - L.ref[3 * tid + 2];
             if (!(dist2(dx, dy, dz) <= hs2)) L.flag[0] = 1;
+            if (two) {   // (left by the first prune; the first step builds whatever they hold)
+                const float qx = static_cast<float>(dx) - L.pr[3 * tid], qy = static_cast<float>(dy) - L.pr[3 * tid + 1];
+                const float qz = static_cast<float>(dz) - L.pr[3 * tid + 2];
+                if (!(fmaf(qz, qz, fmaf(qy, qy, qx * qx)) <= hm2)) L.flag[5] = 1;
+            }
         }
         __syncthreads();
-        if (L.flag[0] != 0) {   // uniform: every thread reads it after the barrier
-            res_build<T>(a, R, S, L);
-            if (tid == 0) res_split(a.tab[blockIdx.x], L);
-            ref[0] = X[0]; ref[1] = X[1]; ref[2] = X[2];
-            if (tid == 0) L.flag[0] = 0;   // read by all before the build's barriers
-            if (own) {   // the build's FP32 positions lay over the force words
-                L.f[3 * tid] = 0;
-                L.f[3 * tid + 1] = 0;
-                L.f[3 * tid + 2] = 0;
+        bool build = L.flag[0] != 0;   // uniform: every thread reads both after the barrier
+        if (build || (two && L.flag[5] != 0)) {
+            for (;;) {
+                if (build) res_build<T>(a, R, S, L, two);
+                res_take<T>(a, R, L, two);
+                if (!two || L.flag[6] == 0) break;   // uniform: read after res_take's barrier
+                two = false;
+                build = true;
+                hs2 = fmin(hs2, 0.25 * kResSkin * kResSkin);
+                __syncthreads();   // every thread has read the flag
+            }
+            if (own) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) {
+                    const double x = L.p[3 * tid + c];
+                    if (build) {
+                        L.ref[3 * tid + c] = x;
+                        L.f[3 * tid + c] = 0;   // the build's FP32 positions lay over the force words
+                    }
+                    L.pr[3 * tid + c] = static_cast<float>(x - L.ref[3 * tid + c]);
+                }
+            }
+            if (tid == 0) {
+                res_split(a.tab[blockIdx.x], L);
+                L.flag[0] = 0;
+                L.flag[5] = 0;
             }
             __syncthreads();
         }
@@ -2806,7 +2917,7 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
             V[1] = half_kick(V[1], S.half_dt, F1 * kFixInv, im);
             V[2] = half_kick(V[2], S.half_dt, F2 * kFixInv, im);
         }
-        a.px[gb] = X[0]; a.py[gb] = X[1]; a.pz[gb] = X[2];
+        a.px[gb] = L.p[3 * tid]; a.py[gb] = L.p[3 * tid + 1]; a.pz[gb] = L.p[3 * tid + 2];
         a.vx[gb] = V[0]; a.vy[gb] = V[1]; a.vz[gb] = V[2];
         a.fx[gb] = F0; a.fy[gb] = F1; a.fz[gb] = F2;
     }
@@ -3165,7 +3276,7 @@ void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host) {
                     d.local_id, d.inv_m, d.res_hs2, d.px, d.py, d.pz,
                     d.vx, d.vy, d.vz, d.f.fx, d.f.fy, d.f.fz, d.res_list, d.fla, d.fld, d.gstep, d.err,
                     d.flags, host, nsteps, d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_excl, d.res_ex_cap,
-                    d.res_units, d.res_unit_cap};
+                    d.res_units, d.res_unit_cap, d.prune_hm2};
     const size_t lds = res_lds_bytes(d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_ex_cap, d.res_unit_cap);
     k_resident<kResThreads><<<d.res_n, kResThreads, lds, st>>>(a);
     if (d.res_n > 1) launch_status_out(d, st, host, nsteps);
