@@ -366,14 +366,6 @@ __device__ __forceinline__ bool baoab_bead_g(const DevSys& S, double im, double 
     return im == 0.0 || (isfinite(x0) && isfinite(x1) && isfinite(x2));
 }
 
-__device__ __forceinline__ bool baoab_bead(const DevSys& S, double im, long long F0, long long F1, long long F2,
-                                           const double (&X)[3], const double (&V)[3], int pending, long long step,
-                                           uint32_t lid, double (&x)[3], double (&v)[3]) {
-    double g[3];
-    gauss3_fast(S.seed, static_cast<uint64_t>(step - S.step_origin), lid, g);
-    return baoab_bead_g(S, im, noise_sigma(S, im), F0, F1, F2, X, V, pending, g, x, v);
-}
-
 // pending != 0: the closing half kick of the previous step is still owed and
 // is applied first.  gstep[pin] is this step's global step; thread 0 writes
 // gstep[pout] = gstep[pin] + 1 for the next step.
@@ -400,14 +392,20 @@ __global__ void k_integrate(int nb, const DevSys* __restrict__ sys, const int* _
     const long long F0 = fx[b], F1 = fy[b], F2 = fz[b];
     const double X0 = px[b], X1 = py[b], X2 = pz[b];
     const double V0 = vx[b], V1 = vy[b], V2 = vz[b];
-    const uint32_t lid = static_cast<uint32_t>(local_id[b]);
+    // the step's noise needs none of them (a single system's local indices are
+    // its beads'): its ~600 cycles run while they are in flight
+    const uint32_t lid = single ? static_cast<uint32_t>(b) : static_cast<uint32_t>(local_id[b]);
+    __builtin_amdgcn_sched_barrier(0);
+    double g[3];
+    gauss3_fast(S.seed, static_cast<uint64_t>(step - S.step_origin), lid, g);
     // an empty statement that needs every loaded value: the loads are all
     // issued before it and waited for once (otherwise the compiler sinks the
     // mobile-bead inputs behind a wait on the mass and a branch)
     asm volatile("" ::"v"(im), "v"(F0), "v"(F1), "v"(F2), "v"(X0), "v"(X1), "v"(X2), "v"(V0), "v"(V1), "v"(V2),
-                 "v"(lid));
+                 "v"(g[0]), "v"(g[1]), "v"(g[2]));
     double xn[3], vn[3];
-    const bool finite = baoab_bead(S, im, F0, F1, F2, {X0, X1, X2}, {V0, V1, V2}, pending, step, lid, xn, vn);
+    const bool finite = baoab_bead_g(S, im, noise_sigma(S, im), F0, F1, F2, {X0, X1, X2}, {V0, V1, V2}, pending, g,
+                                     xn, vn);
     if (!finite) atomicOr(&err[s], kErrNumeric);
     const bool fixed = im == 0.0;
     const double x0 = xn[0], x1 = xn[1], x2 = xn[2], v0 = vn[0], v1 = vn[1], v2 = vn[2];
@@ -1548,7 +1546,6 @@ __device__ inline RowType row_type(const float* __restrict__ t) {
 // constants in the specialized row loops, which then hold no branches; the
 // switch polynomial is evaluated at x = max(0, (r - rsw)/w), where x = 0 gives
 // S = 1 and dS = 0, the unswitched value exactly.
-// (1/r is left in *ir_out when the kinds need it, else 0.)
 // Open Ashbaugh-Hatch groups take s^12 - s^6 and r - rsw from rounded s^12 and
 // r; the periodic loop's fused forms round once less.  Each kind of boundary
 // keeps the rounding its trajectories have always had (OPEN_LJ, a template
@@ -1773,16 +1770,19 @@ struct RowAcc {
     int bad = 0;
 };
 
-// One list entry of a row: the displacement d = x_j - x_i (minimum image
-// applied in place), and g * 2^32 (g = (dE/dr)/r, so that g d is the force on
-// i) in FP64, or 0 when the entry is padding (valid false) or beyond the
-// cutoff.  *bad is set when a pair inside the cutoff exceeded the per-pair
-// limit.  The expression is symmetric in i and j, so the entry (j, i) gives
-// the same g and the negated d.
+// One list entry of a row: its displacement d = x_j - x_i (minimum image
+// applied in place) and f = (dE/dr)/r, so that f d is the force on i; an entry
+// that is padding (valid false) or beyond the cutoff is computed at r2 = 1 and
+// contributes nothing.  The expression is symmetric in i and j, so the entry
+// (j, i) gives the same f and the negated d.
+struct PairF {
+    float f, r2, ir;   // ir: 1/r where the kinds took it (Debye-Hueckel and Ashbaugh-Hatch loops)
+    bool in;
+};
 template <int SPEC>
-__device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const PairK<float>& Kf, const RowType& rt,
-                                             const float* __restrict__ tfj, bool valid, double& dx, double& dy,
-                                             double& dz, int& bad) {
+__device__ __forceinline__ PairF pair_entry(const RowGeom& g, int kinds, const PairK<float>& Kf, const RowType& rt,
+                                            const float* __restrict__ tfj, bool valid, double& dx, double& dy,
+                                            double& dz) {
     // a group without a box has inverse box 0, for which the minimum
     // image is the identity
     if (SPEC == kSpecGeneric || SPEC == kSpecSolo ? g.periodic : !spec_open(SPEC)) {
@@ -1800,26 +1800,50 @@ __device__ __forceinline__ double pair_entry(const RowGeom& g, int kinds, const 
     else if (SPEC == kSpecSolo) f = pair_force(kinds & ~(kExv | kDh | kLjr | kLja), false, Kf.lja_switch, Kf, rt,
                                                tfj, r2f);
     else f = pair_force(kinds & (kExv | kDh | kLjr | kLja), Kf.lj_shared, Kf.lja_switch, Kf, rt, tfj, r2f);
-    // |f d| <= |f| r: one range test covers the three components.  A
-    // pair beyond the limit is flagged and clamped to it along its
-    // direction (so relaxation still pushes the beads apart); NaN
-    // contributes nothing.  Where the kinds already took 1/r the clamp
-    // is formed every time and selected, with no branch in the loop.
-    const bool ok = f * f * r2f < kPairLimit * kPairLimit;
-    bad |= in && !ok;
-    float gg;
+    return {f, r2f, ir, in};
+}
+
+// |f d| <= |f| r: one range test covers the three components.  A pair beyond
+// the limit is flagged and clamped to it along its direction (so relaxation
+// still pushes the beads apart); NaN contributes nothing.  Both are rare: the
+// row loops only test, once for all entries of a round, and come here when a
+// test failed (forming the clamped value for every entry and selecting it took
+// 8 of the ~94 instructions of an Ashbaugh-Hatch entry).
+__device__ __forceinline__ bool pair_over(const PairF& p) { return !(p.f * p.f * p.r2 < kPairLimit * kPairLimit); }
+__device__ __forceinline__ void pair_clamp(PairF& p, int& bad) {
+    if (!pair_over(p)) return;
+    bad |= p.in;
+    p.f = p.f == p.f ? copysignf(0.999f * kPairLimit, p.f) * __builtin_amdgcn_rsqf(p.r2) : 0.0f;
+}
+
+// The same for a loop that handles one entry at a time (resident steps): where
+// the kinds took 1/r anyway the clamped value is selected, without a branch
+// that would split the loop body.
+template <int SPEC>
+__device__ __forceinline__ double pair_scaled_one(const PairF& p, int& bad) {
+    const bool ok = !pair_over(p);
+    bad |= p.in && !ok;
+    float g;
     if (spec_dh(SPEC) || spec_lj(SPEC)) {
-        const float cl = copysignf(0.999f * kPairLimit, f) * ir;
-        gg = ok ? f : (f == f ? cl : 0.0f);
+        const float cl = copysignf(0.999f * kPairLimit, p.f) * p.ir;
+        g = ok ? p.f : (p.f == p.f ? cl : 0.0f);
     } else {
-        gg = ok ? f : (f == f ? copysignf(0.999f * kPairLimit, f) * __builtin_amdgcn_rsqf(r2f) : 0.0f);
+        g = ok ? p.f : (p.f == p.f ? copysignf(0.999f * kPairLimit, p.f) * __builtin_amdgcn_rsqf(p.r2) : 0.0f);
     }
-    gg = in ? gg : 0.0f;   // a masked entry adds exactly the bias constant
-    // scaling by 2^32 is exact in FP32 (the result stays far below
-    // FP32's largest value; a subnormal gg, flushed or not, rounds to
-    // a zero contribution either way), so one FP32 multiply replaces
-    // an FP64 one with the same bits
-    return static_cast<double>(gg * 4294967296.0f);
+    g = p.in ? g : 0.0f;
+    return static_cast<double>(g * 4294967296.0f);
+}
+
+// f * 2^32 in FP64, 0 for an entry that contributes nothing (it then adds
+// exactly the bias constant).  Scaling by 2^32 is exact in FP32 (the result
+// stays far below FP32's largest value; a subnormal f, flushed or not, rounds
+// to a zero contribution either way), so one FP32 multiply replaces an FP64
+// one with the same bits.  The empty statement keeps the selection in front
+// of the conversion, where it is one instruction and not two.
+__device__ __forceinline__ double pair_scaled(const PairF& p) {
+    float g = (p.in ? p.f : 0.0f) * 4294967296.0f;
+    asm("" : "+v"(g));
+    return static_cast<double>(g);
 }
 
 // The kinds of a group whose energy group is in the mask.
@@ -1878,15 +1902,32 @@ __device__ __forceinline__ void force_row(const RowGeom& g, int kinds, const Pai
         // the round's entries are evaluated without branches (an entry that is
         // padding or beyond the cutoff is computed at r2 = 1 and masked to
         // zero) so their dependency chains interleave
+        // (in pairs: two entries' values are what the registers hold beside four records)
+        static_assert(U % 2 == 0, "entries are taken in pairs");
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const PairRec rj = rjs[u];
-            double dx = rj.x - ri.x, dy = rj.y - ri.y, dz = rj.z - ri.z;
-            const float* tfj = lds_types + (rj.type & 0xFFFF) * kTypeStride;
-            const double gs = pair_entry<SPEC>(g, kinds, Kf, rt, tfj, cs[u] >= 0, dx, dy, dz, acc.bad);
-            acc.ux += static_cast<unsigned long long>(__double_as_longlong(fma(gs, dx, kFixMagic)));
-            acc.uy += static_cast<unsigned long long>(__double_as_longlong(fma(gs, dy, kFixMagic)));
-            acc.uz += static_cast<unsigned long long>(__double_as_longlong(fma(gs, dz, kFixMagic)));
+        for (int h = 0; h < U; h += 2) {
+            PairF pf[2];
+            double dx[2], dy[2], dz[2];
+            bool over = false;
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const PairRec rj = rjs[h + u];
+                dx[u] = rj.x - ri.x; dy[u] = rj.y - ri.y; dz[u] = rj.z - ri.z;
+                const float* tfj = lds_types + (rj.type & 0xFFFF) * kTypeStride;
+                pf[u] = pair_entry<SPEC>(g, kinds, Kf, rt, tfj, cs[h + u] >= 0, dx[u], dy[u], dz[u]);
+                over |= pair_over(pf[u]);
+            }
+            if (over) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) pair_clamp(pf[u], acc.bad);
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const double gs = pair_scaled(pf[u]);
+                acc.ux += static_cast<unsigned long long>(__double_as_longlong(fma(gs, dx[u], kFixMagic)));
+                acc.uy += static_cast<unsigned long long>(__double_as_longlong(fma(gs, dy[u], kFixMagic)));
+                acc.uz += static_cast<unsigned long long>(__double_as_longlong(fma(gs, dz[u], kFixMagic)));
+            }
         }
     }
 }
@@ -2665,7 +2706,8 @@ __device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, 
         const double *pi = L.p + bi, *pj = L.p + bj;
         double dx = pj[0] - pi[0], dy = pj[1] - pi[1], dz = pj[2] - pi[2];
         const RowType rt = row_type(L.rows + ti * kTypeStride);
-        const double gs = pair_entry<SPEC>(geo, kinds, Kf, rt, L.rows + tj * kTypeStride, true, dx, dy, dz, bad);
+        const PairF pf = pair_entry<SPEC>(geo, kinds, Kf, rt, L.rows + tj * kTypeStride, true, dx, dy, dz);
+        const double gs = pair_scaled_one<SPEC>(pf, bad);
         const unsigned long long cx =
             static_cast<unsigned long long>(__double_as_longlong(fma(gs, dx, kFixMagic))) - kFixMagicBits;
         const unsigned long long cy =
