@@ -904,7 +904,10 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     d_.res_nbs = (max_n + 63) & ~63;
     // LDS: what one system's step reads, as far as it fits.  Up to one
     // workgroup per CU the whole 160 KB may go to one; beyond that half, so
-    // that two workgroups share a CU and hide each other's latency.
+    // that two workgroups share a CU and hide each other's latency, unless
+    // the part that has to be in LDS is more than half (104 B per bead and
+    // the exclusion tables): then one workgroup per CU (512 chains of 700
+    // beads: 25.6 us/step; 174 on the standard path).
     int max_nt = 0, max_ex = 0;
     long long max_pairs = 0;
     for (int s = 0; s < nsys; ++s) {
@@ -921,13 +924,14 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
         if (hipGetDeviceProperties(&prop, opt_.device) == hipSuccess && prop.multiProcessorCount > 0)
             cus = prop.multiProcessorCount;
     }
-    const size_t budget = (nsys <= cus ? kResLdsMax : kResLdsMax / 2) - 1024;
+    size_t budget = (nsys <= cus ? kResLdsMax : kResLdsMax / 2) - 1024;
     // exclusion tables are staged whole; they are small (chains exclude near
     // neighbours, which are mask bits)
     d_.res_ex_cap = max_ex;
     d_.res_unit_cap = 0;
     for (const ResSys& R : tab) d_.res_unit_cap = std::max(d_.res_unit_cap, R.nu);
     const size_t fixed = resident_lds_bytes(d_.res_nbs, 0, 0, d_.res_ex_cap, d_.res_unit_cap);
+    if (fixed > budget) budget = kResLdsMax - 1024;
     if (fixed > budget) { d_.res_n = 0; return; }
     const size_t room = budget - fixed;
     // half of the list's LDS first, then the terms, then the rest of the list

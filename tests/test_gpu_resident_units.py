@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from opencafemol_amd import abi, configs
-from opencafemol_amd.context import Context
+from opencafemol_amd.context import Batch, Context
 from opencafemol_amd.model import SystemSpec
 
 pytestmark = pytest.mark.gpu
@@ -64,3 +64,22 @@ def test_open_hps_chain():
     s, it, x = configs.hps_open_cluster(6, 100, extent=(5.0, 5.0), seed=2)
     x = x + np.random.default_rng(0).normal(scale=0.005, size=x.shape)
     _both(s, it, x, 5)
+
+
+@pytest.mark.parametrize("n", [640, 704, 1000])
+def test_more_systems_than_cus_with_a_large_one(n):
+    """Beyond one workgroup per CU half the LDS is the limit, and a system that
+    needs more than half takes a CU for itself: it stays resident."""
+    made = [configs.go_chain(n, seed=2)] + [configs.go_chain(5, seed=3)] * 256
+    got = []
+    for resident in (-1, 0):
+        with Batch([m[0] for m in made], [m[1] for m in made], resident=resident) as b:
+            assert (b.resident_threads() > 0) == (resident != 0)
+            for k, (s, it, x) in enumerate(made):
+                b.set_positions(k, x)
+                b.set_velocities(k, np.random.default_rng(k).normal(scale=0.1, size=x.shape))
+            assert b.step(40) == 0
+            got.append([b.state(k, abi.STATE_POSITIONS | abi.STATE_VELOCITIES | abi.STATE_FORCES) for k in (0, 1, 256)])
+    for a, b in zip(*got):
+        for key in ("positions", "velocities", "forces"):
+            assert np.array_equal(a[key], b[key])
