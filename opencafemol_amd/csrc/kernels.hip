@@ -475,7 +475,7 @@ __global__ void k_pack(int nm, const DevPairGroup* __restrict__ groups,
 // cells, which keeps every pair within rl in neighbouring cells.
 // One workgroup per group: the reduction is a chain of gathers (member to bead
 // to position), so 1,024 threads take four members at a time with their loads
-// issued together (21,000 members: 53 us with 256 threads one by one, now 13).
+// issued together (21,000 members: 53 us with 256 threads one by one, now 14).
 constexpr int kOpenGridThreads = 1024;
 __global__ __launch_bounds__(kOpenGridThreads) void k_open_grid(DevPairGroup* __restrict__ groups,
                                                                 const int* __restrict__ member_bead,
