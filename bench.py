@@ -514,7 +514,7 @@ def single_run(args, workload):
     if vf and os.path.exists(vf):
         vj = json.load(open(vf))
         insts = vj["valu_insts_per_entry"] * read_padded
-        # SIMD issue cycles: 4 per wave64 instruction, 8 for an FP64 add/mul/fma
+        # SIMD issue cycles: 4 per wave64 instruction, FP64 like unpacked FP32
         cycles = vj["valu_issue_cycles_per_entry"] * read_padded
         simd_cycles = avg_us * 1e-6 * VALU_CLOCK_HZ * VALU_SIMDS
         valu = {"bound": "valu", "achieved": insts / (avg_us * 1e-6) / 1e9, "peak": VALU_PEAK_GINST,
