@@ -2885,9 +2885,16 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
     // system's entries are one unit or less for each wavefront whatever the
     // skin, and pruning only adds to its step (62 beads: 1.73 us a step with
     // narrow lists, 1.95 pruned; 213 beads: 4.9 and 4.8; 500: 8.6 and 7.1).
-    bool two = R.nb > kResNarrowBeads;   // uniform
+    // A system without pair groups has no list to build or prune: its units are
+    // split once, and it stays out of the loop's list block, whose flags are
+    // cleared behind barriers that only res_build and res_take hold.
+    const bool lists = R.ng > 0;                  // uniform
+    bool two = lists && R.nb > kResNarrowBeads;   // uniform
     if (!two) hs2 = fmin(hs2, 0.25 * kResSkin * kResSkin);
-    if (tid == 0) L.flag[0] = 1;
+    if (tid == 0) {
+        L.flag[0] = 1;
+        if (!lists) res_split(a.tab[blockIdx.x], L);
+    }
     // the FP32 displacement is off by less than 1e-7 nm; the margin's square
     // is reduced by far more
     const float hm2 = static_cast<float>(a.prune_hm2 * (1.0 - 1e-4));
@@ -2919,7 +2926,9 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
             }
         }
         __syncthreads();
-        bool build = L.flag[0] != 0;   // uniform: every thread reads both after the barrier
+        // uniform: every thread reads the flags after the barrier, and they are
+        // written again only behind the barriers of res_build and res_take
+        bool build = lists && L.flag[0] != 0;
         if (build || (two && L.flag[5] != 0)) {
             for (;;) {
                 if (build) res_build<T>(a, R, S, L, two);

@@ -51,12 +51,34 @@ def _only(s, keep):
     return out
 
 
+@pytest.mark.parametrize("n", [70, 300])
 @pytest.mark.parametrize("what", ["bonded", "pairs", "none", "one pair group"])
-def test_partial_sequences(what):
-    s, it, x = configs.go_chain(70, seed=4)
+def test_partial_sequences(what, n):
+    """300 beads: the size that keeps two-level lists where it has pair groups."""
+    s, it, x = configs.go_chain(n, seed=4)
     keep = {"bonded": lambda f: f.kind < abi.EXCLUDED_VOLUME, "pairs": lambda f: f.kind >= abi.EXCLUDED_VOLUME,
             "none": lambda f: False, "one pair group": lambda f: f.kind == abi.DEBYE_HUCKEL}[what]
     _both(_only(s, keep), it, x, 40)
+
+
+def test_bonded_only_beside_pairs():
+    """Without pair groups beside a system that has them: beads move past the
+    batch's prune margin, and there is no list to prune."""
+    made = [configs.go_chain(300, seed=6), configs.go_chain(300, seed=7)]
+    made[0] = (_only(made[0][0], lambda f: f.kind < abi.EXCLUDED_VOLUME),) + made[0][1:]
+    got = []
+    for resident in (-1, 0):
+        with Batch([m[0] for m in made], [m[1] for m in made], resident=resident) as b:
+            assert (b.resident_threads() > 0) == (resident != 0)
+            for k, (s, it, x) in enumerate(made):
+                b.set_positions(k, x)
+                b.set_velocities(k, np.random.default_rng(k).normal(scale=0.3, size=x.shape))
+            for steps in (1, 60, 7):
+                assert b.step(steps) == 0
+            got.append([b.state(k, abi.STATE_POSITIONS | abi.STATE_VELOCITIES | abi.STATE_FORCES) for k in (0, 1)])
+    for a, b in zip(*got):
+        for key in ("positions", "velocities", "forces"):
+            assert np.array_equal(a[key], b[key])
 
 
 def test_open_hps_chain():
