@@ -1190,9 +1190,13 @@ void Engine::layout_rows() {
 }
 
 // After a build reported rows longer than their slots: widen those groups to
-// 1.25x the longest row seen (plus 8) and lay the list out again.
+// 1.25x the longest row seen (plus 8) and lay the list out again.  The new
+// rows hold nothing until the next build.
 void Engine::grow_rows() {
     sync();
+    stale_lists();
+    lists_stale_ = true;
+    list_current_ = false;
     const int ng = static_cast<int>(host_groups_.size());
     std::vector<int> need(std::max(ng, 1), 0);
     check_hip(hipMemcpy(need.data(), d_.group_need, sizeof(int) * need.size(), hipMemcpyDeviceToHost), "need");
@@ -1434,6 +1438,7 @@ int Engine::run_chunk(int k) {
         age_ = p.age1;
         page_ = p.page1;
         fresh_ = 0;
+        if (p.fresh) lists_stale_ = false;   // built in its first step
         for (int s = 0; s < d_.nsys; ++s) {
             if ((err[s] | err_carry_[s]) & kErrNumeric) { sys_status_[s] = OCM_ERR_NUMERIC; numeric = true; }
             err_carry_[s] = 0;
@@ -1727,28 +1732,31 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
     int nrows = 0;
     if ((what & OCM_STATE_POSITIONS) && out->positions) { o.pos = d_.px; dst[nrows++] = out->positions; }
     if ((what & OCM_STATE_VELOCITIES) && out->velocities) { o.vel = d_.vx; dst[nrows++] = out->velocities; }
-    if ((what & OCM_STATE_FORCES) && out->forces) {
-        const uint32_t present = sys_group_mask_[s];
-        ForceBuf src = d_.f;
-        ensure_forces();   // builds (and if needed widens) the list for the current positions
-        if ((present & groups) != present) {
+    const bool forces = (what & OCM_STATE_FORCES) && out->forces;
+    const bool energy = (what & OCM_STATE_ENERGY) != 0;
+    if (forces) ensure_forces();   // builds (and if needed widens) the list for the current positions
+    const uint32_t present = sys_group_mask_[s];
+    const bool subset = forces && (present & groups) != present;
+    // the list the subset's forces and the energies are read from: one build,
+    // before either.  Forces also come from a list within its skin.
+    const bool build = d_.nm > 0 && ((subset && lists_stale_) || (energy && (lists_stale_ || !list_current_)));
+    if (forces) {
+        if (subset) {
             launch_zero_forces(d_, d_.f2, stream_);
-            enqueue_forces(d_.f2, false, groups);
-            src = d_.f2;
+            enqueue_forces(d_.f2, build, groups);
         }
-        o.frc = src.fx;
+        o.frc = subset ? d_.f2.fx : d_.f.fx;
         o.clear_err = 1;   // the full evaluation's flags are carried
         dst[nrows++] = out->forces;
     }
-    if (what & OCM_STATE_ENERGY) {
+    if (build) {
+        if (!subset) { launch_rebuild(d_, stream_); ++rebuilds_; }
+        lists_stale_ = false;
+        list_current_ = true;
+        stale_lists();
+    }
+    if (energy) {
         launch_zero_energy(d_, stream_);
-        if (d_.nm > 0 && (!list_current_ || lists_stale_)) {
-            launch_rebuild(d_, stream_);
-            ++rebuilds_;
-            lists_stale_ = false;
-            list_current_ = true;
-            stale_lists();
-        }
         launch_bonded(d_, stream_, true, d_.f2, groups);
         launch_pair(d_, stream_, true, d_.f2, groups);
         launch_kinetic(d_, stream_);
@@ -1764,10 +1772,9 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
     if (nrows == 0) o.n = 0;
     launch_state_out(stream_, o);
     sync();
-    if ((what & OCM_STATE_ENERGY) && (head_host_[1] & kFlagListOverflow)) {
+    if (energy && (head_host_[1] & kFlagListOverflow)) {
         // the rebuild found a row longer than its slots
         grow_rows();
-        list_current_ = false;
         check_hip(hipMemset(d_.flags, 0, sizeof(int)), "memset");
         get_state(s, what, groups, out);
         return;
@@ -1778,7 +1785,7 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
         if (staged) std::memcpy(dst[k], stage_host_ + 3 * static_cast<size_t>(H.n) * k, bytes);
         else check_hip(hipMemcpy(dst[k], bstate_ + 3 * static_cast<size_t>(H.n) * k, bytes, hipMemcpyDeviceToHost), "state");
     }
-    if (what & OCM_STATE_ENERGY) {
+    if (energy) {
         out->potential_energy = 0;
         for (int g = 0; g < 32; ++g) {
             out->energy_by_group[g] = head_host_[2 + g] * kFixInv;
