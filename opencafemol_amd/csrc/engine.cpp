@@ -1772,8 +1772,8 @@ void Engine::get_state(int s, int what, uint32_t groups, ocm_state* out) {
     if (nrows == 0) o.n = 0;
     launch_state_out(stream_, o);
     sync();
-    if (energy && (head_host_[1] & kFlagListOverflow)) {
-        // the rebuild found a row longer than its slots
+    if (build && (head_host_[1] & kFlagListOverflow)) {
+        // it found a row longer than its slots
         grow_rows();
         check_hip(hipMemset(d_.flags, 0, sizeof(int)), "memset");
         get_state(s, what, groups, out);

@@ -68,3 +68,11 @@ def test_forces_and_energies_when_rows_overflow(oracle, groups):
     with c:
         _check(oracle, s, c, c.get_state(abi.STATE_FORCES | abi.STATE_ENERGY, groups), groups)
         _check(oracle, s, c, c.get_state(abi.STATE_FORCES, CHARGES), CHARGES)
+
+
+@pytest.mark.parametrize("groups", [PAIRS, CHARGES])
+def test_forces_alone_when_rows_overflow(oracle, groups):
+    s, c = _fallen()
+    with c:
+        for _ in range(2):   # the second read reuses the list of the first
+            _check(oracle, s, c, c.get_state(abi.STATE_FORCES, groups), groups)
