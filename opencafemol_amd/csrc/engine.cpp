@@ -1806,7 +1806,6 @@ int Engine::pair_group_of(int s, int force_index) const {
 
 // Rebuilds the outer list at the current positions; returns the flag word.
 int Engine::rebuild_now() {
-    lists_stale_ = false;
     list_current_ = false;
     launch_fill_i32(stream_, d_.flags, 0, 1);
     launch_rebuild(d_, stream_);
@@ -1815,6 +1814,7 @@ int Engine::rebuild_now() {
     sync();
     int flags = 0;
     check_hip(hipMemcpy(&flags, d_.flags, sizeof(int), hipMemcpyDeviceToHost), "flags");
+    lists_stale_ = (flags & kFlagListOverflow) != 0;   // overlong rows are left empty
     return flags;
 }
 

@@ -4,6 +4,7 @@ has a few partners and the slots of the estimate (264 for an open group of 256
 beads or more), and fall into a cube of 1.6 nm, where every row has 599.
 Resident steps do not widen the standard path's rows, so the read does.  Also
 the reads that keep a list between them.  The oracle is the reference."""
+import ctypes as C
 import sys
 
 import numpy as np
@@ -76,3 +77,15 @@ def test_forces_alone_when_rows_overflow(oracle, groups):
     with c:
         for _ in range(2):   # the second read reuses the list of the first
             _check(oracle, s, c, c.get_state(abi.STATE_FORCES, groups), groups)
+
+
+@pytest.mark.parametrize("groups", [PAIRS, CHARGES])
+def test_forces_after_a_refused_noalloc_dump(oracle, groups):
+    """The dump that does not widen rows refuses and leaves a truncated list."""
+    s, c = _fallen()
+    with c:
+        count = C.c_int64(-1)
+        for k in (0, 1):
+            assert c.lib.ocm_get_neighbor_pairs_noalloc(c.h, k, None, 0, C.byref(count)) == abi.OCM_ERR_OOM
+        _check(oracle, s, c, c.get_state(abi.STATE_FORCES, groups), groups)
+        assert c.lib.ocm_get_neighbor_pairs_noalloc(c.h, 0, None, 0, C.byref(count)) == abi.OCM_OK
