@@ -18,7 +18,7 @@ from tests.tolerances import assert_energies_close, assert_forces_close
 pytestmark = pytest.mark.gpu
 
 STEPS, DT = 200, 0.01
-PAIRS, CHARGES = 1, 2   # group masks
+PAIRS, CHARGES, ALL = 1, 2, 0xFFFFFFFF   # group masks
 
 
 @pytest.fixture(autouse=True)
@@ -89,3 +89,28 @@ def test_forces_after_a_refused_noalloc_dump(oracle, groups):
             assert c.lib.ocm_get_neighbor_pairs_noalloc(c.h, k, None, 0, C.byref(count)) == abi.OCM_ERR_OOM
         _check(oracle, s, c, c.get_state(abi.STATE_FORCES, groups), groups)
         assert c.lib.ocm_get_neighbor_pairs_noalloc(c.h, 0, None, 0, C.byref(count)) == abi.OCM_OK
+
+
+@pytest.mark.parametrize("resident", [-1, 0])
+def test_reads_that_keep_a_list_between_them(oracle, resident):
+    """Energies build a list after steps, a subset's forces and energies after
+    them keep it, and new positions or further steps end it."""
+    s, it, x = configs.go_chain(120, seed=9)
+    rng = np.random.default_rng(2)
+    with Context(s, it, resident=resident) as c:
+        c.set_positions(x)
+        c.set_velocities(rng.normal(scale=0.3, size=x.shape))
+        sub = 1 << s.forces[-1].group
+        for new in (None, x + rng.normal(scale=0.02, size=x.shape), None, 3.0 * x):
+            if new is None:
+                assert c.step(150) == abi.OCM_OK
+            else:
+                c.set_positions(new)
+            for what, groups in ((abi.STATE_ENERGY, ALL), (abi.STATE_FORCES, sub), (abi.STATE_ENERGY, sub),
+                                 (abi.STATE_FORCES | abi.STATE_ENERGY, ALL)):
+                st = c.get_state(what | abi.STATE_POSITIONS, groups)
+                F, E = oracle.evaluate(s, st["positions"], groups)
+                if what & abi.STATE_FORCES:
+                    assert_forces_close(st["forces"], F)
+                if what & abi.STATE_ENERGY:
+                    assert_energies_close(st["energy_by_group"], E)
