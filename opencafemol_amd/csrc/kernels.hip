@@ -2346,7 +2346,7 @@ struct ResGroupK {
     int kinds, spec, m0, nm, trow, gid, exo;
     int lds_off, lds_cnt;   // the group's entries kept in LDS: [lds_off, lds_off + lds_cnt)
     int ocnt;               // entries of the last build, in the group's global region
-    int cnt;                // entries the force pass reads
+    int cnt;                // entries the prune kept
     float rl2w, rl2ws;
 };
 
@@ -2379,9 +2379,8 @@ struct ResLds {
     int* lid;          // the beads' indices within their system (noise counters)
     float* rows;
     ResGroupK* gk;
-    int* flag;         // [0] rebuild, [1] FP64 build, [3] where the
-                       // step's units are split, [4] their count, [5] prune, [6] the pruned lists
-                       // did not fit, [8 + g] entries of group g
+    int* flag;         // [0] rebuild, [1] FP64 build, [3] where the step's units are split, [4] their
+                       // count, [5] prune, [8 + g] entries of group g that the force pass reads
     int* ex;           // the system's exclusion tables
     uint32_t* unit;    // the units of its bonded terms
     BTerm* terms;
@@ -2571,35 +2570,72 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
     }
 }
 
-// The entries the force pass reads, from the groups' built lists.  prune: the
-// pairs within cutoff + margin at the positions in LDS, into the groups' shares
-// of the LDS list; flag[6] says that some share was too small.  Otherwise (the
-// pruned lists do not fit): every entry, the first ones of each group in LDS
-// and the rest where the build left them.  All threads call it; it ends with a
-// barrier.  A build costs ~125 k cycles on a 500-bead chain and the entries
-// beyond the cutoff as much as those inside, so lists with a wide skin are
-// built every ~100 steps and pruned every few (~5 k cycles): with one list at
-// 0.3 nm the chain read 2,900 entries a step and built every 31.
-template <int T>
-__device__ void res_take(const ResArgs& a, const ResSys& R, const ResLds& L, bool prune) {
-    const int tid = threadIdx.x, lane = tid & 63;
-    if (R.ng == 0) return;   // uniform
-    if (tid == 0) L.flag[6] = 0;
-    if (tid < R.ng) L.gk[tid].cnt = 0;
-    __syncthreads();
-    long long total = 0;
-    for (int g = 0; g < R.ng; ++g) total += L.gk[g].ocnt;
-    long long before = 0;
+// The groups' shares of the LDS list before a prune, by one thread: what each is
+// expected to keep (flag[8 + g]: what it kept last, or res_guess) and an equal
+// part of the rest.
+__device__ inline void res_shares(const ResSys& R, const ResLds& L, int cap) {
+    int total = 0;
+    for (int g = 0; g < R.ng; ++g) total += L.flag[8 + g];
+    const int spare = max(cap - total, 0) / R.ng;
+    const float scale = total > cap ? 0.999f * static_cast<float>(cap) / static_cast<float>(total) : 1.f;
+    int off = 0;
     for (int g = 0; g < R.ng; ++g) {
-        ResGroupK& K = L.gk[g];
-        const int ocnt = K.ocnt;
-        // a share that holds the whole list while all of them fit, else in proportion
-        const int off = static_cast<int>(total <= a.list_cap ? before : before * a.list_cap / total);
-        before += ocnt;
-        const int room = static_cast<int>(total <= a.list_cap ? before : before * a.list_cap / total) - off;
-        const uint32_t* glist = a.list + K.l0;
-        uint32_t* llist = L.list + off;
-        if (prune) {
+        const int w = L.flag[8 + g];
+        const int room = (total > cap ? static_cast<int>(static_cast<float>(w) * scale) : w) + spare;
+        L.gk[g].lds_off = off;
+        L.gk[g].lds_cnt = room;
+        L.gk[g].cnt = 0;
+        off += room;
+    }
+}
+
+// What the launch's first prune is expected to keep: the built entries by the
+// ratio of the spheres' volumes.
+__device__ inline void res_guess(const ResSys& R, const ResLds& L) {
+    for (int g = 0; g < R.ng; ++g) {
+        const float q = static_cast<float>(L.gk[g].geo.rin2 / L.gk[g].rl2);
+        L.flag[8 + g] = static_cast<int>(static_cast<float>(L.gk[g].ocnt) * q * __builtin_amdgcn_sqrtf(q));
+    }
+}
+
+// The entries the force pass reads, from the groups' built lists.  prune: the
+// pairs within cutoff + margin at the positions in LDS, all of them in the LDS
+// list; false when they do not fit it.  Otherwise: every entry, the first ones
+// in LDS and the rest where the build left them.  All threads call it with a
+// system that has groups; the caller's barrier ends it.
+// A build costs several prunes and the entries beyond the cutoff as much as
+// those inside, so lists with a wide skin are built every ~100 steps and pruned
+// every few.  Groups shrink very differently (a 0.8 nm excluded volume keeps a
+// fifth of its wide list, 3 nm Debye-Hueckel two thirds): shares by the built
+// counts overflowed in one group beside empty space.  A share that is too small
+// after all is made to fit and the prune repeated, so only the total decides.
+template <int T>
+__device__ bool res_take(const ResArgs& a, const ResSys& R, const ResLds& L, bool prune) {
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (!prune) {
+        int off = 0;   // LDS entries of the groups before
+        for (int g = 0; g < R.ng; ++g) {
+            ResGroupK& K = L.gk[g];
+            const int ocnt = K.ocnt, kept = min(ocnt, a.list_cap - off);
+            const uint32_t* glist = a.list + K.l0;
+            for (int e = tid; e < kept; e += T) L.list[off + e] = glist[e];
+            if (tid == 0) {
+                K.lds_off = off;
+                K.lds_cnt = kept;
+                L.flag[8 + g] = ocnt;
+            }
+            off += kept;
+        }
+        return true;
+    }
+    for (;;) {
+        if (tid == 0) res_shares(R, L, a.list_cap);
+        __syncthreads();
+        for (int g = 0; g < R.ng; ++g) {
+            ResGroupK& K = L.gk[g];
+            const int ocnt = K.ocnt, room = K.lds_cnt;
+            const uint32_t* glist = a.list + K.l0;
+            uint32_t* llist = L.list + K.lds_off;
             const RowGeom geo = K.geo;
             for (int e0 = tid; e0 - lane < ocnt; e0 += 4 * T) {   // whole wavefronts
                 uint32_t w[4];
@@ -2626,23 +2662,21 @@ __device__ void res_take(const ResArgs& a, const ResSys& R, const ResLds& L, boo
                     if (keep && at < room) llist[at] = w[k];
                 }
             }
-        } else {
-            for (int e = tid; e < min(ocnt, room); e += T) llist[e] = glist[e];
         }
-        if (tid == 0) {
-            K.lds_off = off;
-            K.lds_cnt = room;   // final below
+        __syncthreads();   // the counts are final
+        int total = 0;
+        bool over = false;
+        for (int g = 0; g < R.ng; ++g) {   // the same for every thread
+            const int c = L.gk[g].cnt;
+            total += c;
+            over |= c > L.gk[g].lds_cnt;
         }
+        if (total > a.list_cap) return false;
+        if (over) __syncthreads();   // the counts have been read
+        if (tid == 0)
+            for (int g = 0; g < R.ng; ++g) L.flag[8 + g] = L.gk[g].cnt;
+        if (!over) return true;
     }
-    __syncthreads();
-    if (tid < R.ng) {
-        ResGroupK& K = L.gk[tid];
-        if (!prune) K.cnt = K.ocnt;
-        if (prune && K.cnt > K.lds_cnt) L.flag[6] = 1;
-        K.lds_cnt = min(K.cnt, K.lds_cnt);
-        L.flag[8 + tid] = K.cnt;
-    }
-    __syncthreads();
 }
 
 // A step's work in units of 64 items (one per lane): the bonded terms, a run
@@ -2932,12 +2966,11 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         if (build || (two && L.flag[5] != 0)) {
             for (;;) {
                 if (build) res_build<T>(a, R, S, L, two);
-                res_take<T>(a, R, L, two);
-                if (!two || L.flag[6] == 0) break;   // uniform: read after res_take's barrier
+                if (s == 0 && two && tid == 0) res_guess(R, L);
+                if (res_take<T>(a, R, L, two)) break;   // uniform
                 two = false;
                 build = true;
                 hs2 = fmin(hs2, 0.25 * kResSkin * kResSkin);
-                __syncthreads();   // every thread has read the flag
             }
             if (own) {
 #pragma unroll
