@@ -934,11 +934,11 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     if (fixed > budget) budget = kResLdsMax - 1024;
     if (fixed > budget) { d_.res_n = 0; return; }
     const size_t room = budget - fixed;
-    // half of the list's LDS first, then the terms, then the rest of the list
+    // kResListLdsFirst entries first, then the terms, then the rest of the list
     const auto list_for = [&](long long most, size_t bytes) {
         return static_cast<int>(std::min<long long>({max_pairs, most, static_cast<long long>(bytes / sizeof(uint32_t))}));
     };
-    const int list_first = list_for(kResListLdsMax / 2, room);
+    const int list_first = list_for(kResListLdsFirst, room);
     d_.res_term_cap = static_cast<int>(std::min<size_t>(static_cast<size_t>(max_nt),
                                                         (room - list_first * sizeof(uint32_t)) / sizeof(BTerm)));
     d_.res_list_cap = list_for(kResListLdsMax, room - d_.res_term_cap * sizeof(BTerm));

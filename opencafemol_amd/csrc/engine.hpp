@@ -179,7 +179,8 @@ private:
     // the next evaluation that reads them rebuilds first
     bool lists_stale_ = false;
     static constexpr int kResChunk = 2000;   // resident steps per launch
-    static constexpr long long kResListLdsMax = 8192;   // list entries per system kept in LDS
+    // list entries per system kept in LDS: before its bonded terms, and in all
+    static constexpr long long kResListLdsFirst = 4096, kResListLdsMax = 16384;
     // host copies of the members' beads and exclusion rows, held while packing
     std::vector<int> excl_bead_, excl_start_h_, excl_count_h_, excl_h_;
     int interval_ = 20;
