@@ -112,10 +112,11 @@ constexpr int kResMaxTypeRows = 64;     // staged type rows per system (6 bits)
 // wrapped into boxes of at most kResWide nm, open systems' relative to bead 0
 // (a build that finds one beyond kResWide tests that build's pairs in FP64).
 constexpr double kResWide = 1000.0;
-// Resident skins (nm, at most): of lists read as built -- every step pays for
-// their width -- and of lists pruned to cutoff + margin between builds.
+// Resident skins (nm, at most): of lists read as built (systems of up to
+// kResNarrowBeads) -- every step pays for their width -- and of lists pruned to
+// cutoff + margin between builds.
 constexpr double kResSkin = 0.3, kResSkinPruned = 0.6;
-constexpr int kResNarrowBeads = 128;   // systems up to this size keep narrow lists
+constexpr int kResNarrowBeads = 128;
 // A unit is up to 64 bonded terms of one kind: bits 0-19 the first term, 20-25
 // the terms less one, 26-31 its cost in kResUnitCost.
 constexpr int kResUnitCost = 16;
@@ -140,12 +141,12 @@ struct ResGroup {
     int gid;          // pair group (DevPairGroup index)
     int m0, nm;       // members [m0, m0 + nm)
     int trow;         // the group's first type row within its system's staged rows
-    long long l0;     // list region: nm (nm - 1) / 2 entries from l0
-    // (cutoff + skin)^2 and the in-kernel build's FP32 threshold (cutoff + skin
-    // + FP32 margin)^2, with the wide skin (lists that are pruned) and the
-    // narrow one (lists read as built)
-    double rl2, rl2s;
-    float rl2w, rl2ws;
+    // list region: nm (nm - 1) / 2 entries from l0; the force pass reads the
+    // entries past the LDS list from r0 on: l0, or as many entries behind it
+    // where the list is pruned
+    long long l0, r0;
+    double rl2;       // (cutoff + resident skin)^2
+    float rl2w;       // (cutoff + skin + FP32 margin)^2: the in-kernel build's threshold
     int exo;          // its exclusion table within the system's: mask [exo, exo + nm),
                       // starts [exo + nm, exo + 2 nm + 1), far partners after them
 };

@@ -879,17 +879,17 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
             }
             // the FP32 thresholds add 1e-3 nm, well above the 2.2e-4 nm error
             // of coordinates below kResWide
-            const double skin = 2.0 * std::sqrt(G.half_skin2);
-            const double skin_w = std::min(skin, kResSkinPruned), skin_n = std::min(skin, kResSkin);
-            Q.rl2 = (G.rc + skin_w) * (G.rc + skin_w);
-            Q.rl2s = (G.rc + skin_n) * (G.rc + skin_n);
-            Q.rl2w = static_cast<float>((G.rc + skin_w + 1e-3) * (G.rc + skin_w + 1e-3));
-            Q.rl2ws = static_cast<float>((G.rc + skin_n + 1e-3) * (G.rc + skin_n + 1e-3));
+            const bool pruned = R.nb > kResNarrowBeads;
+            const double skin = std::min(2.0 * std::sqrt(G.half_skin2), pruned ? kResSkinPruned : kResSkin);
+            Q.rl2 = (G.rc + skin) * (G.rc + skin);
+            Q.rl2w = static_cast<float>((G.rc + skin + 1e-3) * (G.rc + skin + 1e-3));
             for (int i = 0; i < G.member_count; ++i) {
                 double& h = res_hs2[excl_bead_[G.member_begin + i]];
-                h = std::min(h, 0.25 * skin_w * skin_w);
+                h = std::min(h, 0.25 * skin * skin);
             }
-            l0 += std::max<long long>(1, static_cast<long long>(Q.nm) * (Q.nm - 1) / 2);
+            const long long pairs = std::max<long long>(1, static_cast<long long>(Q.nm) * (Q.nm - 1) / 2);
+            Q.r0 = pruned ? l0 + pairs : l0;
+            l0 = Q.r0 + pairs;
             for (int k = 0; k < G.n_types * kTypeStride; ++k)
                 rows.push_back(types_f[static_cast<size_t>(G.type_begin) * kTypeStride + k]);
             trow += G.n_types;

@@ -2341,13 +2341,13 @@ struct ResArgs {
 struct ResGroupK {
     RowGeom geo;
     PairK<float> Kf;
-    long long l0;      // list region in global memory
-    double rl2, rl2s;       // (cutoff + resident skin)^2 with the wide and the narrow skin
+    long long l0, r0;  // list regions in global memory: built, read
+    double rl2;        // (cutoff + resident skin)^2
     int kinds, spec, m0, nm, trow, gid, exo;
     int lds_off, lds_cnt;   // the group's entries kept in LDS: [lds_off, lds_off + lds_cnt)
     int ocnt;               // entries of the last build, in the group's global region
     int cnt;                // entries the prune kept
-    float rl2w, rl2ws;
+    float rl2w;
 };
 
 __host__ __device__ constexpr size_t res_align16(size_t v) { return (v + 15) & ~static_cast<size_t>(15); }
@@ -2411,7 +2411,7 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
 }
 
 // Lists of every group of the system at the positions in LDS, into the groups'
-// global regions, with the wide or the narrow skin.  All threads call it; it
+// global regions.  All threads call it; it
 // overwrites the force words (p32 lies over them) and ends with a barrier,
 // after which they may be written again.
 // The member pairs (i, j > i) are dealt over all threads: rows r and
@@ -2421,7 +2421,7 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
 // mask bit for the next kResNearExcl members, a search of the short sorted
 // list of farther ones, both in LDS).
 template <int T>
-__device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, const ResLds& L, bool wide_skin) {
+__device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, const ResLds& L) {
     const int tid = threadIdx.x;
     if (R.ng == 0) return;   // uniform; nothing is written
     if (tid == 0) L.flag[1] = 0;
@@ -2453,8 +2453,8 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
         const bool wide = L.flag[1] != 0;
         const bool per = K.geo.periodic;
         const int nm = K.nm;
-        const float rl2w = wide_skin ? K.rl2w : K.rl2ws;
-        const double rl2 = wide_skin ? K.rl2 : K.rl2s;
+        const float rl2w = K.rl2w;
+        const double rl2 = K.rl2;
         uint32_t* glist = a.list + K.l0;
         const float Lx = static_cast<float>(G.box[0]), Ly = static_cast<float>(G.box[1]);
         const float Lz = static_cast<float>(G.box[2]);
@@ -2572,7 +2572,10 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
 
 // The groups' shares of the LDS list before a prune, by one thread: what each is
 // expected to keep (flag[8 + g]: what it kept last, or res_guess) and an equal
-// part of the rest.
+// part of the rest.  Groups shrink very differently (a 0.8 nm excluded volume
+// keeps a fifth of its wide list, 3 nm Debye-Hueckel two thirds), so shares by
+// the built counts would leave most of one group's entries outside beside
+// empty space.
 __device__ inline void res_shares(const ResSys& R, const ResLds& L, int cap) {
     int total = 0;
     for (int g = 0; g < R.ng; ++g) total += L.flag[8 + g];
@@ -2599,18 +2602,15 @@ __device__ inline void res_guess(const ResSys& R, const ResLds& L) {
 }
 
 // The entries the force pass reads, from the groups' built lists.  prune: the
-// pairs within cutoff + margin at the positions in LDS, all of them in the LDS
-// list; false when they do not fit it.  Otherwise: every entry, the first ones
-// in LDS and the rest where the build left them.  All threads call it with a
-// system that has groups; the caller's barrier ends it.
+// pairs within cutoff + margin at the positions in LDS, those past the group's
+// share of the LDS list in its second global region.  Otherwise every entry,
+// the first ones in LDS and the rest where the build left them.  All threads
+// call it with a system that has groups; the caller's barrier ends it.
 // A build costs several prunes and the entries beyond the cutoff as much as
 // those inside, so lists with a wide skin are built every ~100 steps and pruned
-// every few.  Groups shrink very differently (a 0.8 nm excluded volume keeps a
-// fifth of its wide list, 3 nm Debye-Hueckel two thirds): shares by the built
-// counts overflowed in one group beside empty space.  A share that is too small
-// after all is made to fit and the prune repeated, so only the total decides.
+// every few.
 template <int T>
-__device__ bool res_take(const ResArgs& a, const ResSys& R, const ResLds& L, bool prune) {
+__device__ void res_take(const ResArgs& a, const ResSys& R, const ResLds& L, bool prune) {
     const int tid = threadIdx.x, lane = tid & 63;
     if (!prune) {
         int off = 0;   // LDS entries of the groups before
@@ -2626,57 +2626,49 @@ __device__ bool res_take(const ResArgs& a, const ResSys& R, const ResLds& L, boo
             }
             off += kept;
         }
-        return true;
+        return;
     }
-    for (;;) {
-        if (tid == 0) res_shares(R, L, a.list_cap);
-        __syncthreads();
-        for (int g = 0; g < R.ng; ++g) {
-            ResGroupK& K = L.gk[g];
-            const int ocnt = K.ocnt, room = K.lds_cnt;
-            const uint32_t* glist = a.list + K.l0;
-            uint32_t* llist = L.list + K.lds_off;
-            const RowGeom geo = K.geo;
-            for (int e0 = tid; e0 - lane < ocnt; e0 += 4 * T) {   // whole wavefronts
-                uint32_t w[4];
+    if (tid == 0) res_shares(R, L, a.list_cap);
+    __syncthreads();
+    for (int g = 0; g < R.ng; ++g) {
+        ResGroupK& K = L.gk[g];
+        const int ocnt = K.ocnt, room = K.lds_cnt;
+        const uint32_t* glist = a.list + K.l0;
+        uint32_t* rest = a.list + K.r0;
+        uint32_t* llist = L.list + K.lds_off;
+        const RowGeom geo = K.geo;
+        for (int e0 = tid; e0 - lane < ocnt; e0 += 4 * T) {   // whole wavefronts
+            uint32_t w[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) w[k] = glist[min(e0 + k * T, ocnt - 1)];
+            for (int k = 0; k < 4; ++k) w[k] = glist[min(e0 + k * T, ocnt - 1)];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    const double *pi = L.p + 3 * (w[k] & 1023), *pj = L.p + 3 * ((w[k] >> 10) & 1023);
-                    double dx = pj[0] - pi[0], dy = pj[1] - pi[1], dz = pj[2] - pi[2];
-                    if (geo.periodic) {
-                        dx = min_image(dx, geo.bx, geo.ibx);
-                        dy = min_image(dy, geo.by, geo.iby);
-                        dz = min_image(dz, geo.bz, geo.ibz);
-                    }
-                    const bool keep = e0 + k * T < ocnt && dist2(dx, dy, dz) < geo.rin2;
-                    const unsigned long long m = __ballot(keep);
-                    if (m == 0ull) continue;   // the same for the wavefront
-                    int base = 0;
-                    if (lane == 0) base = atomicAdd(&K.cnt, __popcll(m));
-                    base = __builtin_amdgcn_readfirstlane(base);
-                    const int at = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-                                              static_cast<uint32_t>(m >> 32),
-                                              __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
-                    if (keep && at < room) llist[at] = w[k];
+            for (int k = 0; k < 4; ++k) {
+                const double *pi = L.p + 3 * (w[k] & 1023), *pj = L.p + 3 * ((w[k] >> 10) & 1023);
+                double dx = pj[0] - pi[0], dy = pj[1] - pi[1], dz = pj[2] - pi[2];
+                if (geo.periodic) {
+                    dx = min_image(dx, geo.bx, geo.ibx);
+                    dy = min_image(dy, geo.by, geo.iby);
+                    dz = min_image(dz, geo.bz, geo.ibz);
+                }
+                const bool keep = e0 + k * T < ocnt && dist2(dx, dy, dz) < geo.rin2;
+                const unsigned long long m = __ballot(keep);
+                if (m == 0ull) continue;   // the same for the wavefront
+                int base = 0;
+                if (lane == 0) base = atomicAdd(&K.cnt, __popcll(m));
+                base = __builtin_amdgcn_readfirstlane(base);
+                const int at = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                          static_cast<uint32_t>(m >> 32),
+                                          __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
+                if (keep) {
+                    if (at < room) llist[at] = w[k];
+                    else rest[at] = w[k];
                 }
             }
         }
-        __syncthreads();   // the counts are final
-        int total = 0;
-        bool over = false;
-        for (int g = 0; g < R.ng; ++g) {   // the same for every thread
-            const int c = L.gk[g].cnt;
-            total += c;
-            over |= c > L.gk[g].lds_cnt;
-        }
-        if (total > a.list_cap) return false;
-        if (over) __syncthreads();   // the counts have been read
-        if (tid == 0)
-            for (int g = 0; g < R.ng; ++g) L.flag[8 + g] = L.gk[g].cnt;
-        if (!over) return true;
     }
+    __syncthreads();   // the counts are final
+    if (tid == 0)
+        for (int g = 0; g < R.ng; ++g) L.flag[8 + g] = L.gk[g].cnt;
 }
 
 // A step's work in units of 64 items (one per lane): the bonded terms, a run
@@ -2729,7 +2721,7 @@ __device__ inline void res_split(const ResSys& R, const ResLds& L) {
 template <int SPEC, int T>
 __device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, int beg, int end, int cnt,
                                           ResDeal<T / 64>& D, const ResLds& L, int& bad) {
-    const uint32_t* glist = a.list + K.l0;
+    const uint32_t* glist = a.list + K.r0;
     const uint32_t* llist = L.list + K.lds_off;
     const int lcnt = K.lds_cnt;
     const RowGeom geo = K.geo;
@@ -2758,7 +2750,7 @@ __device__ __forceinline__ void res_pairs(const ResArgs& a, const ResGroupK& K, 
         atomicAdd(Fj + 2, 0ull - cz);
     };
     // entries kept in LDS, the rest read through a buffer resource over the
-    // group's global region (a different load than LDS's, so neither becomes
+    // group's read region (a different load than LDS's, so neither becomes
     // a generic load, and the entry body is inlined once)
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint32_t*>(glist), 0, cnt * static_cast<int>(sizeof(uint32_t)), 0x00020000);
@@ -2896,6 +2888,7 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
                         G.periodic != 0};
         K.Kf = pair_constants<float>(G);
         K.l0 = Q.l0;
+        K.r0 = Q.r0;
         K.kinds = G.kinds;
         K.spec = pair_spec(G.kinds, G.periodic != 0, K.Kf);
         K.m0 = Q.m0;
@@ -2904,27 +2897,24 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         K.gid = Q.gid;
         K.exo = Q.exo;
         K.rl2 = Q.rl2;
-        K.rl2s = Q.rl2s;
         K.lds_off = 0;
         K.lds_cnt = 0;
         K.ocnt = 0;
         K.cnt = 0;
         K.rl2w = Q.rl2w;
-        K.rl2ws = Q.rl2ws;
     }
     if (tid < 8 + kResMaxGroups) L.flag[tid] = 0;
     __syncthreads();
-    // lists: built wide and pruned, or, once the pruned lists did not fit the
-    // LDS list, built narrow and taken whole; the first step builds.  A small
-    // system's entries are one unit or less for each wavefront whatever the
-    // skin, and pruning only adds to its step (62 beads: 1.73 us a step with
-    // narrow lists, 1.95 pruned; 213 beads: 4.9 and 4.8; 500: 8.6 and 7.1).
+    // lists: built wide and pruned, or, up to kResNarrowBeads, built narrow and
+    // read as built; the first step builds.  A small system's entries are one
+    // unit or less for each wavefront whatever the skin, and pruning only adds
+    // to its step (62 beads: 1.73 us a step with narrow lists, 1.95 pruned; 213
+    // beads: 4.9 and 4.8; 500: 8.6 and 7.1).
     // A system without pair groups has no list to build or prune: its units are
     // split once, and it stays out of the loop's list block, whose flags are
     // cleared behind barriers that only res_build and res_take hold.
     const bool lists = R.ng > 0;                  // uniform
-    bool two = lists && R.nb > kResNarrowBeads;   // uniform
-    if (!two) hs2 = fmin(hs2, 0.25 * kResSkin * kResSkin);
+    const bool two = lists && R.nb > kResNarrowBeads;   // uniform
     if (tid == 0) {
         L.flag[0] = 1;
         if (!lists) res_split(a.tab[blockIdx.x], L);
@@ -2962,16 +2952,12 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         __syncthreads();
         // uniform: every thread reads the flags after the barrier, and they are
         // written again only behind the barriers of res_build and res_take
-        bool build = lists && L.flag[0] != 0;
-        if (build || (two && L.flag[5] != 0)) {
-            for (;;) {
-                if (build) res_build<T>(a, R, S, L, two);
-                if (s == 0 && two && tid == 0) res_guess(R, L);
-                if (res_take<T>(a, R, L, two)) break;   // uniform
-                two = false;
-                build = true;
-                hs2 = fmin(hs2, 0.25 * kResSkin * kResSkin);
-            }
+        const bool build = lists && L.flag[0] != 0;
+        if (__builtin_expect(build || (two && L.flag[5] != 0), 0)) {
+            const ResSys& Q = a.tab[blockIdx.x];
+            if (build) res_build<T>(a, Q, a.sys[Q.sys], L);
+            if (s == 0 && two && tid == 0) res_guess(Q, L);
+            res_take<T>(a, Q, L, two);
             if (own) {
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {

@@ -111,7 +111,11 @@ std::size_t Server::estimate_bytes(const HostSystem& s) const {
         const double list_bytes = opt_.engine.prune_interval > 1 ? 8.0 : 4.0;   // outer (+ inner) list
         bytes += s.n * (list_bytes * per_bead + 48.0) + 8.0 * f.exclusions.size();
     }
-    // a resident-sized system's own list holds every member pair (4 bytes each)
+    // a resident-sized system's own lists hold every member pair of a group (4
+    // bytes each, above kResNarrowBeads twice).  One group's pairs once are
+    // counted: with the rows counted for every bead above, chains and slabs of
+    // 500 to 1,000 beads take 63-91% of the estimate, a 648-bead membrane
+    // patch with four groups 1.5 times it (6.7 MB).
     if (s.n <= kResMaxBeads) bytes += 2.0 * s.n * s.n;
     return static_cast<std::size_t>(bytes) + (1u << 20);
 }

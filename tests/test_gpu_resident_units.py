@@ -30,7 +30,8 @@ def _both(s, it, x, steps):
             assert (c.resident_threads() > 0) == (resident != 0)
             c.set_positions(x)
             c.set_velocities(v)
-            assert c.step(steps) == 0
+            for n in steps if isinstance(steps, tuple) else (steps,):
+                assert c.step(n) == 0
             st = c.get_state(abi.STATE_POSITIONS | abi.STATE_VELOCITIES | abi.STATE_FORCES)
             got.append((st["positions"], st["velocities"], st["forces"], st["step"]))
     for a, b in zip(*got):
@@ -86,6 +87,22 @@ def test_open_hps_chain():
     s, it, x = configs.hps_open_cluster(6, 100, extent=(5.0, 5.0), seed=2)
     x = x + np.random.default_rng(0).normal(scale=0.005, size=x.shape)
     _both(s, it, x, 5)
+
+
+@pytest.mark.parametrize("what", ["cluster", "slab", "lipids"])
+def test_pruned_lists_past_the_lds(what):
+    """Dense systems whose pruned lists pass the LDS list (16,384 entries at
+    most): open Ashbaugh-Hatch and Debye-Hueckel groups, the periodic ones, and
+    four groups of the membrane kinds; calls of several lengths."""
+    s, it, x = {"cluster": lambda: configs.hps_open_cluster(7, 140, extent=(5.0, 5.0), seed=1),
+                "slab": lambda: configs.hps_slab(n_chains=10, chain_len=100, box=(8.0, 8.0, 60.0), slab_z=15.0, seed=1),
+                "lipids": lambda: configs.lipid_patch(216, box=(6.0, 6.0, 9.0), spacing=1.0, seed=1)}[what]()
+    with Context(s, it) as c:
+        c.set_positions(x + np.random.default_rng(0).normal(scale=0.005, size=x.shape))
+        c.minimize(50.0, 200)
+        x = c.get_state(abi.STATE_POSITIONS)["positions"]
+    for steps in ((80,), (1, 30, 49)):
+        _both(s, it, x, steps)
 
 
 @pytest.mark.parametrize("n", [640, 704, 1000])
