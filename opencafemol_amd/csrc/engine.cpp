@@ -926,12 +926,18 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     }
     size_t budget = (nsys <= cus ? kResLdsMax : kResLdsMax / 2) - 1024;
     // exclusion tables are staged whole; they are small (chains exclude near
-    // neighbours, which are mask bits)
+    // neighbours, which are mask bits).  Where they do not fit beside the beads
+    // (1,000 beads in 7 or more groups, or in 2 with 6 far exclusions a bead), the
+    // builds of a batch read them from memory; a few systems alone are faster
+    // on the standard path.
     d_.res_ex_cap = max_ex;
     d_.res_unit_cap = 0;
     for (const ResSys& R : tab) d_.res_unit_cap = std::max(d_.res_unit_cap, R.nu);
-    const size_t fixed = resident_lds_bytes(d_.res_nbs, 0, 0, d_.res_ex_cap, d_.res_unit_cap);
-    if (fixed > budget) budget = kResLdsMax - 1024;
+    const auto fixed_part = [&] { return resident_lds_bytes(d_.res_nbs, 0, 0, d_.res_ex_cap, d_.res_unit_cap); };
+    if (fixed_part() > budget) budget = kResLdsMax - 1024;
+    d_.res_ex_lds = !(fixed_part() > budget && nsys >= kResTableBatch);
+    if (!d_.res_ex_lds) d_.res_ex_cap = 0;
+    const size_t fixed = fixed_part();
     if (fixed > budget) { d_.res_n = 0; return; }
     const size_t room = budget - fixed;
     // kResListLdsFirst entries first, then the terms, then the rest of the list
@@ -943,7 +949,7 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
                                                         (room - list_first * sizeof(uint32_t)) / sizeof(BTerm)));
     d_.res_list_cap = list_for(kResListLdsMax, room - d_.res_term_cap * sizeof(BTerm));
     const size_t lds = resident_lds_bytes(d_.res_nbs, d_.res_term_cap, d_.res_list_cap, d_.res_ex_cap, d_.res_unit_cap);
-    check_hip(resident_prepare(lds), "hipFuncSetAttribute (resident LDS)");
+    check_hip(resident_prepare(d_, lds), "hipFuncSetAttribute (resident LDS)");
     d_.res_tab = dalloc<ResSys>(tab.size()); upload(d_.res_tab, tab);
     d_.res_grp = dalloc<ResGroup>(std::max<size_t>(grp.size(), 1));
     if (!grp.empty()) upload(d_.res_grp, grp);

@@ -179,6 +179,11 @@ private:
     // the next evaluation that reads them rebuilds first
     bool lists_stale_ = false;
     static constexpr int kResChunk = 2000;   // resident steps per launch
+    // Systems from which exclusion tables may stay in memory (1,000 beads in 8
+    // groups, us per step of 16 / 24 / 256 systems: 37 / 37 / 40, standard path
+    // 31 / 41 / 389; in 2 groups with 6 far exclusions a bead 15 / 14 / 15,
+    // standard 16 / 20 / 151).
+    static constexpr int kResTableBatch = 24;
     // list entries per system kept in LDS: before its bonded terms, and in all
     static constexpr long long kResListLdsFirst = 4096, kResListLdsMax = 16384;
     // host copies of the members' beads and exclusion rows, held while packing

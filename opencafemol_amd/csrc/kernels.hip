@@ -2419,8 +2419,9 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
 // into S segments so that about 2T segments cover the group; a thread tests
 // its segments' candidates one after another against the row's exclusions (a
 // mask bit for the next kResNearExcl members, a search of the short sorted
-// list of farther ones, both in LDS).
-template <int T>
+// list of farther ones).
+// EX_LDS: the exclusion tables are staged in LDS (otherwise read from memory).
+template <int T, bool EX_LDS>
 __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, const ResLds& L) {
     const int tid = threadIdx.x;
     if (R.ng == 0) return;   // uniform; nothing is written
@@ -2463,7 +2464,7 @@ __device__ void res_build(const ResArgs& a, const ResSys& R, const DevSys& S, co
         const int nrp = (nm + 1) / 2;                       // row pairs
         const int nseg = max(1, (2 * T + nrp - 1) / max(nrp, 1));   // segments per row pair
         const int seglen = (nm - 1 + nseg - 1) / nseg;
-        const int* exm = L.ex + K.exo;
+        const int* exm = EX_LDS ? L.ex + K.exo : a.excl_tab + R.ex0 + K.exo;
         const int* far = exm + 2 * nm + 1;
         // consecutive threads take different row pairs: the entries one wave
         // appends together (consecutive list slots, read together by a wave of
@@ -2837,7 +2838,7 @@ __device__ __forceinline__ void res_forces(const ResArgs& a, const ResSys& R, co
 // velocities are synchronized (no half kick owed); on exit the same holds
 // nsteps later.  Every barrier is reached by every thread: the step count
 // and the rebuild decision (read from LDS after a barrier) are uniform.
-template <int T>
+template <int T, bool EX_LDS>
 __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char res_base[];
     const ResLds L = res_lds(res_base, a.nbs, a.term_cap, a.ex_cap, a.unit_cap);
@@ -2878,7 +2879,8 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         int* dst = reinterpret_cast<int*>(L.terms);
         for (int k = tid; k < nw; k += T) dst[k] = src[k];
     }
-    for (int k = tid; k < R.exn; k += T) L.ex[k] = a.excl_tab[R.ex0 + k];
+    if (EX_LDS)
+        for (int k = tid; k < R.exn; k += T) L.ex[k] = a.excl_tab[R.ex0 + k];
     for (int k = tid; k < R.nu; k += T) L.unit[k] = a.units[R.u0 + k];
     if (tid < R.ng) {
         const ResGroup Q = a.grp[R.g0 + tid];
@@ -2955,7 +2957,7 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
         const bool build = lists && L.flag[0] != 0;
         if (__builtin_expect(build || (two && L.flag[5] != 0), 0)) {
             const ResSys& Q = a.tab[blockIdx.x];
-            if (build) res_build<T>(a, Q, a.sys[Q.sys], L);
+            if (build) res_build<T, EX_LDS>(a, Q, a.sys[Q.sys], L);
             if (s == 0 && two && tid == 0) res_guess(Q, L);
             res_take<T>(a, Q, L, two);
             if (own) {
@@ -3336,8 +3338,15 @@ size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap, int u
     return res_lds_bytes(nbs, term_cap, list_cap, ex_cap, unit_cap);
 }
 
-hipError_t resident_prepare(size_t lds) {
-    return hipFuncSetAttribute(reinterpret_cast<const void*>(&k_resident<kResThreads>), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+// The instance for batches whose exclusion tables are in LDS, or in memory.
+static const void* resident_kernel(bool ex_lds) {
+    return ex_lds ? reinterpret_cast<const void*>(&k_resident<kResThreads, true>)
+                  : reinterpret_cast<const void*>(&k_resident<kResThreads, false>);
+}
+
+hipError_t resident_prepare(const DevPtrs& d, size_t lds) {
+    return hipFuncSetAttribute(resident_kernel(d.res_ex_lds), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               static_cast<int>(lds));
 }
 
 void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host) {
@@ -3348,7 +3357,8 @@ void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host) {
                     d.flags, host, nsteps, d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_excl, d.res_ex_cap,
                     d.res_units, d.res_unit_cap, d.prune_hm2};
     const size_t lds = res_lds_bytes(d.res_nbs, d.res_term_cap, d.res_list_cap, d.res_ex_cap, d.res_unit_cap);
-    k_resident<kResThreads><<<d.res_n, kResThreads, lds, st>>>(a);
+    if (d.res_ex_lds) k_resident<kResThreads, true><<<d.res_n, kResThreads, lds, st>>>(a);
+    else k_resident<kResThreads, false><<<d.res_n, kResThreads, lds, st>>>(a);
     if (d.res_n > 1) launch_status_out(d, st, host, nsteps);
 }
 

@@ -81,7 +81,8 @@ struct DevPtrs {
     int res_n = 0, res_threads = 0;
     int res_term_cap = 0, res_list_cap = 0;   // bonded terms and list entries held in LDS per system
     int res_nbs = 0;                          // LDS entries per bead array (multiple of 64)
-    int res_ex_cap = 0;                       // exclusion-table words per system (staged in LDS)
+    int res_ex_cap = 0;                       // LDS words for a system's exclusion tables
+    bool res_ex_lds = true;                   // the tables are staged there, else read from memory
     int* res_excl = nullptr;
     int res_unit_cap = 0;                     // words of a system's unit table (staged in LDS)
     uint32_t* res_units = nullptr;
@@ -158,7 +159,7 @@ void launch_resident(const DevPtrs& d, hipStream_t st, int nsteps, int* host);
 // LDS of one resident workgroup (bead arrays of nbs entries), and the
 // attribute that allows it (gfx950 gives a workgroup up to 160 KB).
 size_t resident_lds_bytes(int nbs, int term_cap, int list_cap, int ex_cap, int unit_cap);
-hipError_t resident_prepare(size_t lds);
+hipError_t resident_prepare(const DevPtrs& d, size_t lds);
 // One workgroup size: a step's units are dealt over all of its wavefronts.
 constexpr int kResThreads = 1024;
 constexpr size_t kResLdsMax = 160 * 1024;

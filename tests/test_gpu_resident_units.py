@@ -122,3 +122,29 @@ def test_more_systems_than_cus_with_a_large_one(n):
     for a, b in zip(*got):
         for key in ("positions", "velocities", "forces"):
             assert np.array_equal(a[key], b[key])
+
+
+@pytest.mark.parametrize("count", [23, 24])
+def test_exclusion_tables_that_do_not_fit(count):
+    """1,000 beads with six exclusions beyond the mask bits for each bead and
+    nonbonded force: the tables do not fit the LDS, and batches of 24 systems
+    and more read them from memory (fewer step on the standard path)."""
+    s, it, x = configs.go_chain(1000, seed=3)
+    i = np.arange(960)
+    far = np.concatenate([np.stack([i, i + 34 + k], 1) for k in range(6)]).astype(np.int32)
+    for f in s.forces:
+        if f.kind >= abi.EXCLUDED_VOLUME:
+            f.category, f.n_categories = np.zeros(s.n, np.int32), 1   # every bead takes part
+            f.exclusions = np.concatenate([np.asarray(f.exclusions, np.int32).reshape(-1, 2), far])
+    got = []
+    for resident in (-1, 0):
+        with Batch([s] * count, [it] * count, resident=resident) as b:
+            assert (b.resident_threads() > 0) == (resident != 0 and count >= 24)
+            for k in range(count):
+                b.set_positions(k, x)
+                b.set_velocities(k, np.random.default_rng(k).normal(scale=0.1, size=x.shape))
+            assert b.step(60) == 0
+            got.append([b.state(k, abi.STATE_POSITIONS | abi.STATE_VELOCITIES | abi.STATE_FORCES) for k in (0, count - 1)])
+    for a, b in zip(*got):
+        for key in ("positions", "velocities", "forces"):
+            assert np.array_equal(a[key], b[key])
