@@ -636,7 +636,7 @@ void Engine::pack() {
     {
         // pinned, device-mapped and coherent: the chunk's last kernel writes
         // the status words straight into it; behind them the head of a state
-        // read and the staging of its arrays.  Up to 1 MiB is staged (14,000
+        // read and the staging of its arrays.  Up to 1 MiB is staged (21,845
         // beads' positions and velocities): past that the host's copy out of
         // the staging costs more than the runtime's own copy to the caller.
         void* h = nullptr;
@@ -907,7 +907,7 @@ void Engine::pack_resident(const std::vector<BTerm>& terms, const std::vector<De
     // that two workgroups share a CU and hide each other's latency, unless
     // the part that has to be in LDS is more than half (104 B per bead and
     // the exclusion tables): then one workgroup per CU (512 chains of 700
-    // beads: 25.6 us/step; 174 on the standard path).
+    // beads: 19.1 us/step; 174 on the standard path).
     int max_nt = 0, max_ex = 0;
     long long max_pairs = 0;
     for (int s = 0; s < nsys; ++s) {

@@ -1031,7 +1031,7 @@ template <typename R> struct V3T { R x, y, z; };
 // reads are one wait: a wavefront with one term per lane has nothing else to
 // hide them behind (with a branch and a wait per vector, the dihedral
 // wavefront that bounds a 62-bead chain's step took 3.7 k cycles; with the
-// units dealt from two ends the step went from 2.54 to 1.73 us).
+// units dealt from two ends the step went from 2.59 to 1.92 us).
 template <int N>
 __device__ __forceinline__ void bdisps(const double* __restrict__ px, const double* __restrict__ py,
                                        const double* __restrict__ pz, const int (&from)[N], const int (&to)[N],
@@ -2207,8 +2207,8 @@ __global__ __launch_bounds__(kPairBlock) __attribute__((amdgpu_waves_per_eu(5)))
 // and atomics on one word are served one at a time (~12 ns each).  With one
 // atomic per table entry, wavefront and kind on a single copy the pass took
 // 116 us on the 14,000-bead slab (9,000 in a row on a word), and forces and
-// energies of a frame 736 us; with the kinetic sums spread the same way the
-// frame takes 519 us.
+// energies of a frame 736 us; with the kinetic sums spread the same way 519 us
+// (227 with its state read in one launch and the list kept).
 template <int TEAM>
 __global__ __launch_bounds__(kPairBlock) void k_pair_energy(
     const DevPairGroup* __restrict__ groups, const int4* __restrict__ blocks, const PairRec* __restrict__ rec,
@@ -2299,7 +2299,7 @@ __global__ __launch_bounds__(kPairBlock) void k_pair_energy(
 // same bits as the standard path.
 // Everything a step reads sits in LDS where it fits (gfx950 gives a
 // workgroup up to 160 KB): the system's bonded terms up to term_cap, its list
-// up to list_cap entries (the rest stays in global memory), the groups'
+// up to list_cap entries (the rest is in global memory), the groups'
 // constants and type rows.  A step is two barriers: the integrator (thread b
 // steps bead b), then the force pass, whose work -- bonded terms, list
 // entries, and the next step's noise of every bead -- is dealt out as one
@@ -2411,9 +2411,8 @@ __device__ __forceinline__ ResLds res_lds(unsigned char* base, int nbs, int term
 }
 
 // Lists of every group of the system at the positions in LDS, into the groups'
-// global regions.  All threads call it; it
-// overwrites the force words (p32 lies over them) and ends with a barrier,
-// after which they may be written again.
+// global regions.  All threads call it; it overwrites the force words (p32 lies
+// over them) and ends with a barrier, after which they may be written again.
 // The member pairs (i, j > i) are dealt over all threads: rows r and
 // nm - 1 - r together hold nm - 1 candidates, and each such row pair is cut
 // into S segments so that about 2T segments cover the group; a thread tests
@@ -2910,8 +2909,9 @@ __global__ __launch_bounds__(T) void k_resident(ResArgs a) {
     // lists: built wide and pruned, or, up to kResNarrowBeads, built narrow and
     // read as built; the first step builds.  A small system's entries are one
     // unit or less for each wavefront whatever the skin, and pruning only adds
-    // to its step (62 beads: 1.73 us a step with narrow lists, 1.95 pruned; 213
-    // beads: 4.9 and 4.8; 500: 8.6 and 7.1).
+    // to its step (us a step with narrow lists and pruned: Go chains of 62 beads
+    // 1.92 and 2.11, 128: 2.93 and 2.61, 213: 4.14 and 3.82, 500: 7.65 and 6.69;
+    // AICG2+ chains of 62: 2.07 and 2.25, 128: 3.46 and 3.55, 213: 5.58 and 5.29).
     // A system without pair groups has no list to build or prune: its units are
     // split once, and it stays out of the loop's list block, whose flags are
     // cleared behind barriers that only res_build and res_take hold.
